@@ -87,6 +87,9 @@ constexpr int kQmmMaxRows = kPrefillChunk;
 bool qmm_supported(const QWeight& w);
 int qmm(const QWeight& w, const uint16_t* x, int64_t x_stride, int m, const ProjEpilogue& e,
         hipStream_t s);
+// qmm beyond 16 rows (gemm.hip); arguments as qmm has checked them
+int qmm_gemm(const QWeight& w, const uint16_t* x, int64_t x_stride, int m, const ProjEpilogue& e,
+             hipStream_t s);
 // exact-integer projections for 1..8 rows (xq.hip): the CPU oracle's
 // mxo_xq arithmetic bit for bit, on the int8 matrix cores
 // plane (nullable): the activation operands of x, written by its producer in

@@ -175,304 +175,6 @@ void dense_bits(const QWeight& w, const uint16_t* x, int64_t xs, int m, const Pr
 }
 
 // ---------------------------------------------------------------------------
-// Prefill GEMM (more than 16 activation rows): a workgroup computes a tile of
-// 64 weight rows x 128 activation rows over the groups [g0, g1) of its k
-// slice (blockIdx.z); wave (wn, wm) of its 2 x 2 waves owns 32 weight rows
-// (two 16-row tiles) x 64 activation rows (four 16-row tiles).  The
-// activations of two groups (128 k) at a time are staged in LDS once for the
-// four waves (eight lanes per 128-byte row piece), and so are the weights of
-// those groups, dequantised (gemm_dq_kernel); the next two groups'
-// activations are in flight while the matrix cores work on these, and the
-// weights of the stage after are requested too.  With a k split the
-// workgroups write fp32 partials and gemm_reduce_kernel adds them in slice
-// order before the epilogue.
-constexpr int kGemmM = 128;          // activation rows per workgroup
-constexpr int kGemmN = 64;           // weight rows per workgroup
-constexpr int kGemmLd = 64 + 8;      // padded LDS row (bf16) of one group
-constexpr int kGemmStage = 2;        // groups staged per barrier pair
-
-// The projection epilogues of one output (activation row m, weight row `row`).
-__device__ __forceinline__ void gemm_epilogue(const ProjEpilogue& e, int n, int m, int row,
-                                              float v) {
-  if (e.mode == kPlain) {
-    e.y[size_t(m) * e.y_stride + row] = f32_to_bf16(v);
-  } else if (e.mode == kHcDown) {
-    const float tt = round_bf16(round_bf16(v) / float(e.hc));
-    if (row < e.rank)
-      e.y[size_t(m) * e.y_stride + row] = f32_to_bf16(tt * sigmoid_bf16(tt));
-    else
-      e.aux[size_t(m) * e.aux_stride + (row - e.rank)] = f32_to_bf16(sigmoid_bf16(tt) * 2.0f);
-  } else {  // kHcWrite
-    const float vb = round_bf16(v);
-    for (int s = 0; s < e.hc; ++s) {
-      uint16_t* res = e.y + size_t(m) * e.y_stride + size_t(s) * n + row;
-      const float inj = round_bf16(vb * bf16_to_f32(e.aux[size_t(m) * e.aux_stride + s]));
-      *res = f32_to_bf16(bf16_to_f32(*res) + inj);
-    }
-  }
-}
-
-// Prefill projections: the weights dequantised once per workgroup.  Each
-// stage, thread t turns 32 codes of weight row t / 4 (k piece t % 4 of the
-// stage's 128; BITS 32-bit words) into w = s q + b in fp32 and stores two bf16 parts in LDS,
-// hi = bf16(w) and lo = bf16(w - hi) (w - hi is exact in fp32; hi + lo is w
-// to within 2^-17 |w|).  The waves then multiply plain tiles, x hi + x lo
-// into fp32 accumulators over the whole slice, with no per-group scale work
-// per output (the exact-code form applies s and b to every output of every
-// group, and its 128 q offset cancels in fp32).  Lane quarter kq of MFMA step
-// st covers k = 16 kq + 8 st .. + 7 of a group on both operands.
-constexpr int kDqLd = 2 * 64 + 8;  // padded LDS row (bf16) of a stage's weights
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-__host__ __device__ constexpr int gemm_dq_lds() {
-  return (kGemmStage * kGemmM * kGemmLd + 2 * kGemmN * kDqLd) * 2;
-}
-
-// Code v (0..31) of a 32-code piece held in BITS words, value v at bit BITS v.
-template <int BITS, int V>
-__device__ __forceinline__ uint32_t piece_code(const uint32_t (&w)[BITS]) {
-  constexpr int bit = BITS * V, word = bit >> 5, off = bit & 31;
-  constexpr uint32_t mask = (1u << BITS) - 1u;
-  if constexpr (off + BITS <= 32)
-    return (w[word] >> off) & mask;
-  else
-    return __builtin_amdgcn_alignbit(w[word + 1], w[word], uint32_t(off)) & mask;
-}
-
-// MIX (kHcUpMix, no k split): the workgroup's 64 weight rows are the four
-// streams' rows s H + c of 16 columns c (blockIdx.x 16 .. + 15), and the
-// epilogue mixes the four streams of each column through LDS with
-// dense_kernel's kHcUpMix arithmetic.
-template <int BITS, bool SPLIT, bool MIX = false>
-__global__ __launch_bounds__(256) void gemm_dq_kernel(QWeight w, const uint16_t* __restrict__ x,
-                                                      int64_t x_stride, int M, int per,
-                                                      ProjEpilogue e) {
-  extern __shared__ __align__(16) uint16_t dq_lds[];
-  auto xs = reinterpret_cast<uint16_t (*)[kGemmM][kGemmLd]>(dq_lds);
-  auto wh = reinterpret_cast<uint16_t (*)[kDqLd]>(dq_lds + kGemmStage * kGemmM * kGemmLd);
-  auto wl = wh + kGemmN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j = lane & 15, kq = lane >> 4;
-  const int wn = wave & 1, wm = wave >> 1;
-  const int n = w.n, G = w.k >> 6;
-  const int mb = blockIdx.y * kGemmM;
-  const int gbeg = blockIdx.z * per;
-  const int gend = min(G, gbeg + per);
-  // dequantising role: weight row dr of the workgroup, 32-value piece dp
-  const int dr = tid >> 2, dp = tid & 3;
-  const int cb = int(blockIdx.x) * 16;  // MIX: the workgroup's first column
-  const int wrow = MIX ? (dr >> 4) * e.hidden + min(cb + (dr & 15), e.hidden - 1)
-                       : min(int(blockIdx.x) * kGemmN + dr, n - 1);
-  const uint32_t* crow = w.codes + size_t(wrow) * (size_t(w.k) * BITS / 32);
-  const uint16_t* srow = w.scales + size_t(wrow) * G;
-  const uint16_t* brow = w.biases + size_t(wrow) * G;
-  const int sc8 = tid & 7, sr0 = tid >> 3;
-  uint4 xv[8];
-  auto load_x = [&](int g0) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = sr0 + 32 * (i & 3), g = g0 + (i >> 2);
-      if (mb + r < M && g < gend)
-        xv[i] = *reinterpret_cast<const uint4*>(x + size_t(mb + r) * x_stride + 64 * g + 8 * sc8);
-      else
-        xv[i] = make_uint4(0u, 0u, 0u, 0u);
-    }
-  };
-  struct StageW {
-    uint32_t c[BITS];  // 32 codes of row dr, group g0 + dp / 2, half dp % 2
-    uint16_t sc, bi;
-  };
-  auto load_w = [&](int g0, StageW& st) {
-    const int g = min(g0 + (dp >> 1), gend - 1);
-    const uint32_t* src = crow + 2 * BITS * g + BITS * (dp & 1);
-    if constexpr (BITS % 4 == 0) {  // 16-byte aligned pieces
-#pragma unroll
-      for (int i = 0; i < BITS / 4; ++i) {
-        const uint4 v = reinterpret_cast<const uint4*>(src)[i];
-        st.c[4 * i] = v.x;
-        st.c[4 * i + 1] = v.y;
-        st.c[4 * i + 2] = v.z;
-        st.c[4 * i + 3] = v.w;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < BITS; ++i) st.c[i] = src[i];
-    }
-    st.sc = srow[g];
-    st.bi = brow[g];
-  };
-  floatx4_t y[2][4];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) y[t][u] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  StageW w0, w1;
-  load_w(gbeg, w0);
-  load_w(gbeg + kGemmStage, w1);
-  load_x(gbeg);
-  for (int g0 = gbeg; g0 < gend; g0 += kGemmStage) {
-    StageW w2;
-    load_w(g0 + 2 * kGemmStage, w2);  // two stages ahead (clamped to the slice)
-    __syncthreads();                  // every wave is done with the previous stage's LDS
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = sr0 + 32 * (i & 3), gs = i >> 2;
-      *reinterpret_cast<uint4*>(&xs[gs][r][8 * sc8]) = xv[i];
-    }
-    {
-      const float sc = bf16_to_f32(w0.sc), bi = bf16_to_f32(w0.bi);
-      uint32_t qv[32];
-      [&]<int... V>(std::integer_sequence<int, V...>) {
-        ((qv[V] = piece_code<BITS, V>(w0.c)), ...);
-      }(std::make_integer_sequence<int, 32>{});
-#pragma unroll
-      for (int q8 = 0; q8 < 4; ++q8) {  // codes 8 q8 .. + 7
-        uint32_t hw[4], lw[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float v0 = fmaf_(sc, float(qv[8 * q8 + 2 * i]), bi);
-          const float v1 = fmaf_(sc, float(qv[8 * q8 + 2 * i + 1]), bi);
-          const bf16x2_t h = {__bf16(v0), __bf16(v1)};
-          const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-          const bf16x2_t l = {__bf16(v0 - u2f(hb << 16)), __bf16(v1 - u2f(hb & 0xffff0000u))};
-          hw[i] = hb;
-          lw[i] = __builtin_bit_cast(uint32_t, l);
-        }
-        const int col = 32 * dp + 8 * q8;
-        *reinterpret_cast<uint4*>(&wh[dr][col]) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-        *reinterpret_cast<uint4*>(&wl[dr][col]) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-      }
-    }
-    __syncthreads();
-    if (g0 + kGemmStage < gend) load_x(g0 + kGemmStage);  // next stage, in flight
-#pragma unroll
-    for (int s = 0; s < kGemmStage; ++s) {
-      if (g0 + s >= gend) break;  // uniform
-      uint4 bh[2][2], bl[2][2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          const int nr = wn * 32 + 16 * t + j, col = 64 * s + 16 * kq + 8 * st;
-          bh[t][st] = *reinterpret_cast<const uint4*>(&wh[nr][col]);
-          bl[t][st] = *reinterpret_cast<const uint4*>(&wl[nr][col]);
-        }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int row = wm * 64 + 16 * u + j;
-        const uint4* xp = reinterpret_cast<const uint4*>(&xs[s][row][16 * kq]);
-        const uint4 a0 = xp[0], a1 = xp[1];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          y[t][u] = mfma_bf16(a0, bh[t][0], y[t][u]);
-          y[t][u] = mfma_bf16(a1, bh[t][1], y[t][u]);
-          y[t][u] = mfma_bf16(a0, bl[t][0], y[t][u]);
-          y[t][u] = mfma_bf16(a1, bl[t][1], y[t][u]);
-        }
-      }
-    }
-    w0 = w1;
-    w1 = w2;
-  }
-  if constexpr (MIX) {
-    // stream s = 2 wn + t of column cb + j: bf16(p) into LDS [row][s][column]
-    __syncthreads();  // the last stage's operands are read
-    float* ex = reinterpret_cast<float*>(dq_lds);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          ex[((wm * 64 + 16 * u + 4 * kq + r) * 4 + 2 * wn + t) * 16 + j] = round_bf16(y[t][u][r]);
-    __syncthreads();
-    for (int i = tid; i < kGemmM * 16; i += 256) {
-      const int ml = i >> 4, c = i & 15, m = mb + ml;
-      if (m >= M || cb + c >= e.hidden) continue;
-      float sum = 0.0f;
-#pragma unroll
-      for (int st = 0; st < 4; ++st) {
-        const float xn =
-            bf16_to_f32(e.xn[size_t(m) * e.xn_stride + size_t(st) * e.hidden + cb + c]);
-        sum = sum + round_bf16(sigmoid_bf16(ex[(ml * 4 + st) * 16 + c]) * xn);
-      }
-      e.y[size_t(m) * e.y_stride + cb + c] = f32_to_bf16(round_bf16(sum) / 4.0f);
-    }
-    return;
-  }
-  const int nb = blockIdx.x * kGemmN + wn * 32;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = nb + 16 * t + j;
-    if (row >= n) continue;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = mb + wm * 64 + 16 * u + 4 * kq + r;
-        if (m >= M) continue;
-        if constexpr (SPLIT)
-          e.part[(size_t(blockIdx.z) * M + m) * n + row] = y[t][u][r];
-        else
-          gemm_epilogue(e, n, m, row, y[t][u][r]);
-      }
-  }
-}
-
-// The k slices' partial sums added in slice order, then the epilogue.
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(int n, int M, int slices,
-                                                          ProjEpilogue e) {
-  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= size_t(M) * n) return;
-  const int m = int(i / n), row = int(i - size_t(m) * n);
-  float v = e.part[i];
-  for (int z = 1; z < slices; ++z) v = v + e.part[size_t(z) * M * n + i];
-  gemm_epilogue(e, n, m, row, v);
-}
-
-template <int BITS>
-void launch_gemm(const QWeight& w, const uint16_t* x, int64_t xs, int m, const ProjEpilogue& e,
-                 hipStream_t s) {
-  const int G = w.k >> 6;
-  const int mb = (m + kGemmM - 1) / kGemmM;
-  if (e.mode == kHcUpMix) {  // four streams of 16 columns per workgroup, no k split
-    const void* fn = reinterpret_cast<const void*>(gemm_dq_kernel<BITS, false, true>);
-    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dq_lds()) !=
-        hipSuccess)
-      return;
-    hipLaunchKernelGGL((gemm_dq_kernel<BITS, false, true>), dim3((e.hidden + 15) / 16, mb, 1),
-                       dim3(256), gemm_dq_lds(), s, w, x, xs, m, G, e);
-    return;
-  }
-  const int nb = (w.n + kGemmN - 1) / kGemmN;
-  // split k across workgroups until the grid has about 256 workgroups, each
-  // slice at least four groups, when the workspace holds the partials
-  int slices = 1;
-  while (nb * mb * slices < 256 && G / (2 * slices) >= 4 && e.part &&
-         size_t(2 * slices) * m * w.n <= e.part_floats)
-    slices *= 2;
-  const int per = (G + slices - 1) / slices;
-  const dim3 grid(nb, mb, slices);
-  // the LDS above the default 64 KiB needs the kernel attribute
-  const void* fn = slices == 1 ? reinterpret_cast<const void*>(gemm_dq_kernel<BITS, false>)
-                               : reinterpret_cast<const void*>(gemm_dq_kernel<BITS, true>);
-  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dq_lds()) !=
-      hipSuccess)
-    return;
-  if (slices == 1)
-    hipLaunchKernelGGL((gemm_dq_kernel<BITS, false>), grid, dim3(256), gemm_dq_lds(), s, w, x,
-                       xs, m, per, e);
-  else
-    hipLaunchKernelGGL((gemm_dq_kernel<BITS, true>), grid, dim3(256), gemm_dq_lds(), s, w, x,
-                       xs, m, per, e);
-  if (slices > 1) {
-    const size_t outs = size_t(m) * w.n;
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3(unsigned((outs + 255) / 256)), dim3(256), 0, s,
-                       w.n, m, slices, e);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Experts.  One workgroup serves one plan entry (an expert and the rows that
 // chose it) for 4/SK tile groups.  gate/up: NT = 2 (the gate tile and the up
 // tile of the same 16 rows), SwiGLU in the epilogue.  down: NT = 1, the route
@@ -831,15 +533,7 @@ int qmm(const QWeight& w, const uint16_t* x, int64_t x_stride, int m, const Proj
   if (!qmm_supported(w) || m < 1 || m > kQmmMaxRows) return MX_EUNSUPPORTED;
   if (e.mode == kHcUpMix && e.hidden * 4 != w.n) return MX_EUNSUPPORTED;
   if (e.mode == kConv) return MX_EUNSUPPORTED;
-  if (m > 16) {  // prefill rows: the staged GEMM
-    switch (w.bits) {
-      case 4: launch_gemm<4>(w, x, x_stride, m, e, s); break;
-      case 5: launch_gemm<5>(w, x, x_stride, m, e, s); break;
-      case 6: launch_gemm<6>(w, x, x_stride, m, e, s); break;
-      default: launch_gemm<8>(w, x, x_stride, m, e, s); break;
-    }
-    return hipGetLastError() == hipSuccess ? MX_OK : MX_EHIP;
-  }
+  if (m > 16) return qmm_gemm(w, x, x_stride, m, e, s);  // prefill rows (gemm.hip)
   switch (w.bits) {
     case 4: dense_bits<4>(w, x, x_stride, m, e, s); break;
     case 5: dense_bits<5>(w, x, x_stride, m, e, s); break;
