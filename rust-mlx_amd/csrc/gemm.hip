@@ -258,7 +258,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_deep_kernel(QWeight w,
 // (padded rows measured 8 % slower).  A group at a time instead of two halves
 // the LDS and the registers: three to four workgroups per CU overlap one's
 // barriers and dequantising with another's matrix-core work.  512 x 12352 x
-// 2048, 4 bits: 64 us (UW = 8), 100 us with two groups per stage at two
+// 2048, 4 bits: 61 us (UW = 8), 91 us with two groups per stage at two
 // workgroups per CU.
 // MIX (kHcUpMix): the 64 weight rows are the four streams' rows s H + c of 16
 // columns c, mixed through LDS in the epilogue (dense_kernel's arithmetic).
@@ -374,6 +374,18 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(QWeight w, const uint16_
       }
       e.y[size_t(m) * e.y_stride + cb + c] = f32_to_bf16(round_bf16(sum) / 4.0f);
     }
+  } else if (!SPLIT && e.mode == kPlain) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int row = int(blockIdx.x) * 64 + wn * 32 + 16 * t + j;
+#pragma unroll
+      for (int u = 0; u < UW; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = mb + wm * 16 * UW + 16 * u + 4 * kq + r;
+          if (m < M && row < n) e.y[size_t(m) * e.y_stride + row] = f32_to_bf16(y[t][u][r]);
+        }
+    }
   } else {
     // sixteen rows at a time through this wave's own part of LDS, so that a
     // row's 32 outputs are written together
@@ -418,7 +430,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(int n, int M, int slic
 // (the other widths differ by a few per cent and keep the order):
 //  tile  4 + groups * 0.125 (UW + 1.5) * rounds, rounds = workgroups / 256
 //        halfway rounded up and at least 1.35 (a lone workgroup per CU has
-//        nothing to overlap its barriers with): 64 us at 512 x 12352 x 2048
+//        nothing to overlap its barriers with): 61 us at 512 x 12352 x 2048
 //        (UW 8; 72 at UW 4), 57 us at 512 x 9216 x 2048 (UW 4; 64 at UW 8),
 //        23 us at 300 x 20000 x 512 (UW 4; 32 at UW 8).
 //  split tile  the same over groups / slices, plus the reduction's launch and
