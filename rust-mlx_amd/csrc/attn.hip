@@ -460,18 +460,36 @@ __global__ __launch_bounds__(kMaxHd) void combine_kernel(const float* __restrict
   }
 }
 
+constexpr int kPfKeys = 64;  // keys per tile of the prefill kernel
+// Keys of one split of a query block that attends to `keys` keys in at most
+// `splits` splits: whole tiles, every split but the last full.
+__device__ __forceinline__ int prefill_split_len(int keys, int splits) {
+  const int tiles = (keys + kPfKeys - 1) / kPfKeys;
+  return (tiles + splits - 1) / splits * kPfKeys;
+}
+
+// The largest position of the query block of qb (<= 64) rows at qb0.
+__device__ __forceinline__ int block_max_pos(const int32_t* __restrict__ pos, int qb0, int qb,
+                                             int rows) {
+  const int lane = threadIdx.x & 63;
+  int v = lane < qb && qb0 + lane < rows ? pos[qb0 + lane] : -1;
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
 // Fast-mode combine (matrix-core decode partials, 64-position chunks): the
 // chunk weights w_c = e^(m_c - M) are formed once per chunk by threads c and
 // shared through LDS (hardware exp2); L = sum_c l_c w_c as a block sum;
 // O[d] = sum_c o_c[d] w_c (fma, c ascending); y = bf16(bf16(O / L) * sigmoid(gate)).
-// chunks <= 256 (max_ctx <= 16384, checked on the host).
+// chunks <= 256 (max_ctx <= 16384, checked on the host).  qb > 0: the prefill
+// kernel's partials, `chunk_len` splits of query blocks of qb rows.
 __global__ __launch_bounds__(256) void combine_fast_kernel(const float* __restrict__ o_part,
                                                            const float* __restrict__ ml_part,
                                                            const uint16_t* __restrict__ qkv,
                                                            int64_t qkv_stride,
                                                            const int32_t* __restrict__ pos,
                                                            AttnDims d, int max_chunks,
-                                                           int chunk_len,
+                                                           int chunk_len, int qb,
                                                            uint16_t* __restrict__ out) {
   __shared__ float wsh[256];
   __shared__ float red[2][4];
@@ -479,6 +497,8 @@ __global__ __launch_bounds__(256) void combine_fast_kernel(const float* __restri
   const int row = blockIdx.y;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int hd = d.head_dim;
+  if (qb > 0)
+    chunk_len = prefill_split_len(block_max_pos(pos, row / qb * qb, qb, gridDim.y) + 1, chunk_len);
   const int chunks = (pos[row] + chunk_len) / chunk_len;
   const float* ml = ml_part + (size_t(row) * d.heads + h) * max_chunks * 2;
   const float* op = o_part + (size_t(row) * d.heads + h) * max_chunks * hd + min(t, hd - 1);
@@ -521,7 +541,7 @@ __global__ __launch_bounds__(256) void combine_fast_kernel(const float* __restri
 // ---------------------------------------------------------------------------
 // Prefill attention on the matrix cores (fast mode, a chunk of query rows of
 // one slot): a workgroup of eight waves takes QB = 8 * 16 / G query rows, one
-// kv head and one split of kPfSplit key positions, so the key and value rows
+// kv head and one split of the key positions, so the key and value rows
 // of a tile are read once for all QB rows x G heads.  Wave w owns one M tile
 // of 16 (row, head) pairs: pair i = row qb0 + w * 16 / G + i / G, head
 // kvh * G + i % G.  Per tile of kPfKeys keys: K rows and V (transposed) are
@@ -531,11 +551,26 @@ __global__ __launch_bounds__(256) void combine_fast_kernel(const float* __restri
 // through LDS into A-operand order as two bf16 parts (hi + lo), and O += P V
 // on the matrix cores (fp32 accumulators, rescaled by e^(m_old - m_new)).
 // The split's (m, l, O) per pair go to o_part / ml_part at chunk index =
-// split, which combine_fast_kernel merges with chunk length kPfSplit.  Rows of
+// split, which combine_fast_kernel merges.  Rows of
 // one query block must share a slot (a prefill chunk's rows do).
-constexpr int kPfKeys = 64;     // keys per tile
-constexpr int kPfSplit = 256;   // keys per split (one partial per pair and split)
-static_assert(attn_prefill_splits(kPfSplit + 1) == 2, "attn_prefill_splits counts kPfSplit keys");
+// max / sum over the 16 lanes of a row by rotations (no LDS)
+template <int ROT>
+__device__ __forceinline__ float row_ror(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + ROT, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, row_ror<8>(v));
+  v = fmaxf(v, row_ror<4>(v));
+  v = fmaxf(v, row_ror<2>(v));
+  return fmaxf(v, row_ror<1>(v));
+}
+__device__ __forceinline__ float row_sum(float v) {
+  v = v + row_ror<8>(v);
+  v = v + row_ror<4>(v);
+  v = v + row_ror<2>(v);
+  return v + row_ror<1>(v);
+}
 constexpr int kPfKLd = kMaxHd + 8;      // padded K row in LDS (bf16)
 constexpr int kPfVLd = kPfKeys + 8;     // padded transposed-V row (bf16)
 
@@ -558,18 +593,13 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
   uint16_t* ks = pf_lds;                              // [kPfKeys][kPfKLd]
   uint16_t* vt = ks + kPfKeys * kPfKLd;               // [HD][kPfVLd]
   uint16_t* pw = vt + HD * kPfVLd;                    // [8 waves][hi, lo][16][kPfVLd]
-  __shared__ int blk_max;
   const int split = blockIdx.x, kvh = blockIdx.y, qb0 = blockIdx.z * QB;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int j = lane & 15, kq = lane >> 4;
-  if (t == 0) {
-    int mx = -1;
-    for (int r = qb0; r < min(qb0 + QB, rows); ++r) mx = max(mx, pos[r]);
-    blk_max = mx;
-  }
-  __syncthreads();
-  const int key0 = split * kPfSplit;
-  const int kend = min(key0 + kPfSplit, blk_max + 1);  // keys [key0, kend)
+  const int blk_max = block_max_pos(pos, qb0, QB, rows);
+  const int len = prefill_split_len(blk_max + 1, gridDim.x);
+  const int key0 = split * len;
+  const int kend = min(key0 + len, blk_max + 1);  // keys [key0, kend)
   if (key0 >= kend) return;                             // uniform
   const size_t base = size_t(slots[qb0]) * d.slot_stride + size_t(kvh) * d.max_ctx * HD;
   // this lane's A-operand pair (j) and the D-layout pairs 4 kq + r
@@ -672,9 +702,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
         sc[c][r] = v ? sc[c][r] * sl2 : u2f(0xff800000u);
         mt = fmaxf(mt, sc[c][r]);
       }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) mt = fmaxf(mt, __shfl_xor(mt, off, 64));
-      const float mn = fmaxf(m_run[r], mt);
+      const float mn = fmaxf(m_run[r], row_max(mt));
       const bool none = mn == u2f(0xff800000u);  // no valid key yet
       const float alpha = none || m_run[r] == u2f(0xff800000u)
                               ? 0.0f
@@ -688,9 +716,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
         sc[c][r] = pv;
         ls += pv;
       }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) ls += __shfl_xor(ls, off, 64);
-      l_run[r] = l_run[r] * alpha + ls;
+      l_run[r] = l_run[r] * alpha + ls;  // this lane's keys; the lanes' sums are added at the end
       m_run[r] = mn;
 #pragma unroll
       for (int n = 0; n < NO; ++n) o[n][r] *= alpha;
@@ -706,7 +732,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
         ph[(4 * kq + r) * kPfVLd + 16 * c + j] = __builtin_bit_cast(uint16_t, h);
         pl[(4 * kq + r) * kPfVLd + 16 * c + j] = __builtin_bit_cast(uint16_t, __bf16(pv - hf));
       }
-    __syncthreads();
+    __builtin_amdgcn_wave_barrier();  // P is this wave's own
     // O += P V: A = P (pair j, keys 32 s + 8 kq ..), B = V^T rows (dim 16 n + j)
 #pragma unroll
     for (int st = 0; st < kPfKeys / 32; ++st) {
@@ -726,6 +752,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
   for (int r = 0; r < 4; ++r) {
     const int i = 4 * kq + r;
     const int row = qb0 + wave * RPW + i / G;
+    const float l = row_sum(l_run[r]);
     if (row >= rows) continue;
     const size_t ph_ = (size_t(row) * d.heads + kvh * G + i % G) * max_chunks + split;
 #pragma unroll
@@ -733,7 +760,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
     if (j == 0) {
       // m in natural-log units, as the decode kernels write it
       ml_part[ph_ * 2] = m_run[r] * 0.6931471805599453f;
-      ml_part[ph_ * 2 + 1] = l_run[r];
+      ml_part[ph_ * 2 + 1] = l;
     }
   }
 }
@@ -805,7 +832,7 @@ int attn_combine(const float* o_part, const float* ml_part, const uint16_t* qkv,
   if (fast) {
     if ((d.max_ctx + kAttnFastChunk - 1) / kAttnFastChunk > 256) return MX_EUNSUPPORTED;
     hipLaunchKernelGGL(combine_fast_kernel, dim3(d.heads, rows), dim3(256), 0, s, o_part,
-                       ml_part, qkv, qkv_stride, pos, d, max_chunks, kAttnFastChunk, out);
+                       ml_part, qkv, qkv_stride, pos, d, max_chunks, kAttnFastChunk, 0, out);
   } else {
     const bool pl = plane && rows <= 8 && d.head_dim % xq::kGroup == 0;
     hipLaunchKernelGGL(combine_kernel, dim3(d.heads, rows), dim3(kMaxHd), 0, s, o_part, ml_part,
@@ -819,15 +846,31 @@ bool attn_prefill_supported(AttnDims d) {
   if (!attn_fast_supported(d)) return false;
   const int g = d.heads / d.kv_heads;
   return (d.head_dim == 256 || d.head_dim == 128) && (g == 2 || g == 4 || g == 8) &&
-         (d.max_ctx + kPfSplit - 1) / kPfSplit <= 256;
+         attn_prefill_splits(d.max_ctx) <= 256;
 }
+
+namespace {
+constexpr int prefill_block_rows(int g) { return 8 * 16 / g; }
+// Splits of each query block's keys: as many workgroups as CUs (107 KB of LDS
+// lets one run per CU), within the partials' room.  Every split costs its 128
+// pairs a partial of fp32 sums, written and read: 509 rows at positions 1500
+// .. 2008, 16 heads on 2: 61 us with 4 splits, 127 us with 256-key splits
+// (sized by the cache, so half of the workgroups had no keys; the softmax also
+// reduced through LDS and the waves met for P).
+int prefill_splits(int rows, AttnDims d, int max_chunks) {
+  const int qb = prefill_block_rows(d.heads / d.kv_heads);
+  const int blocks = (rows + qb - 1) / qb * d.kv_heads;
+  const int want = 256 / blocks, room = max_chunks < 256 ? max_chunks : 256;
+  return want < 1 ? 1 : want < room ? want : room;
+}
+}  // namespace
 
 int attn_prefill(const uint16_t* q, int rows, const int32_t* slots, const int32_t* pos,
                  const uint16_t* k_cache, const uint16_t* v_cache, AttnDims d, int max_chunks,
                  float* o_part, float* ml_part, hipStream_t s) {
   if (!attn_prefill_supported(d)) return MX_EUNSUPPORTED;
-  const int splits = (d.max_ctx + kPfSplit - 1) / kPfSplit;
-  if (splits > max_chunks) return MX_EINVAL;
+  if (attn_prefill_splits(d.max_ctx) > max_chunks) return MX_EINVAL;
+  const int splits = prefill_splits(rows, d, max_chunks);
   const float scale = 1.0f / __builtin_sqrtf(float(d.head_dim));
   const int g = d.heads / d.kv_heads;
 #define MX_PF(GG, HH)                                                                        \
@@ -837,7 +880,7 @@ int attn_prefill(const uint16_t* q, int rows, const int32_t* slots, const int32_
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn),                               \
                             hipFuncAttributeMaxDynamicSharedMemorySize, lb) != hipSuccess)   \
       return MX_EHIP;                                                                        \
-    constexpr int qb = 8 * 16 / GG;                                                          \
+    constexpr int qb = prefill_block_rows(GG);                                               \
     hipLaunchKernelGGL(fn, dim3(splits, d.kv_heads, (rows + qb - 1) / qb), dim3(512), lb, s, \
                        q, rows, slots, pos, k_cache, v_cache, d, max_chunks, scale, o_part,  \
                        ml_part);                                                             \
@@ -851,9 +894,10 @@ int attn_prefill(const uint16_t* q, int rows, const int32_t* slots, const int32_
 int attn_combine_splits(const float* o_part, const float* ml_part, const uint16_t* qkv,
                         int64_t qkv_stride, int rows, const int32_t* pos, AttnDims d,
                         int max_chunks, uint16_t* out, hipStream_t s) {
-  if ((d.max_ctx + kPfSplit - 1) / kPfSplit > 256) return MX_EUNSUPPORTED;
+  if (attn_prefill_splits(d.max_ctx) > 256) return MX_EUNSUPPORTED;
   hipLaunchKernelGGL(combine_fast_kernel, dim3(d.heads, rows), dim3(256), 0, s, o_part, ml_part,
-                     qkv, qkv_stride, pos, d, max_chunks, kPfSplit, out);
+                     qkv, qkv_stride, pos, d, max_chunks, prefill_splits(rows, d, max_chunks),
+                     prefill_block_rows(d.heads / d.kv_heads), out);
   return hipGetLastError() == hipSuccess ? MX_OK : MX_EHIP;
 }
 

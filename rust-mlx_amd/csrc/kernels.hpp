@@ -195,8 +195,9 @@ int attn_combine(const float* o_part, const float* ml_part, const uint16_t* qkv,
 constexpr int kAttnChunk = 256;
 constexpr int kAttnFastChunk = 64;
 // Prefill (fast mode): query rows of one slot in blocks that share each key
-// tile, one partial per (row, head) and split of 256 keys at chunk index =
-// split; attn_combine_splits merges them (and applies the output gate).
+// tile, one partial per (row, head) and split of the keys at chunk index =
+// split (at most attn_prefill_splits(max_ctx) are asked of max_chunks);
+// attn_combine_splits merges them (and applies the output gate).
 bool attn_prefill_supported(AttnDims d);
 constexpr int attn_prefill_splits(int max_ctx) { return (max_ctx + 255) / 256; }
 int attn_prefill(const uint16_t* q, int rows, const int32_t* slots, const int32_t* pos,

@@ -114,3 +114,38 @@ def test_attn_prefill_form_within_tolerance(mx, orc, heads, kv_heads, hd, p0, ro
         assert np.all(np.abs(g - ref) <= 2.0 ** -6 * np.abs(ref) + 2.0 ** -9 * scale), flags
     a, b = bf(got[1]).astype(np.float64), bf(got[3]).astype(np.float64)
     assert np.all(np.abs(a - b) <= 2.0 ** -6 * np.abs(ref) + 2.0 ** -9 * scale)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,p0,rows,max_ctx", [
+    (16, 2, 256, 0, 300, 320), (8, 1, 128, 1800, 9, 2000), (4, 2, 128, 60, 200, 300),
+    (32, 8, 128, 500, 512, 1024), (8, 2, 256, 1000, 1, 1024)])
+def test_attn_prefill_splits_of_every_kind(mx, orc, heads, kv_heads, hd, p0, rows, max_ctx):
+    """The prefill form where its keys split otherwise: one split for each query
+    block (many blocks), as many as the partials hold (few rows), blocks of
+    fewer tiles than splits, chunks from position 0, a single row; against the
+    float64 closed form with the matrix-core kernel's bound."""
+    rng = np.random.default_rng(heads * 100 + rows)
+    pos = np.arange(p0, p0 + rows, dtype=np.int32)
+    slots = np.zeros(rows, np.int32)
+    kc, vc = (orc.f32_to_bf16(rng.standard_normal((1, kv_heads, max_ctx, hd)).astype(np.float32))
+              for _ in range(2))
+    q = orc.f32_to_bf16((rng.standard_normal((rows, heads, hd)) * 0.3).astype(np.float32))
+    qkv = orc.f32_to_bf16(rng.standard_normal((rows, 2 * heads * hd)).astype(np.float32))
+    G = heads // kv_heads
+    k64, v64 = (bf(np.repeat(a[0], G, axis=0)).astype(np.float64) for a in (kc, vc))
+    s = np.einsum("rhd,hnd->hrn", bf(q).astype(np.float64), k64) / np.sqrt(hd)
+    s[:, np.arange(max_ctx)[None, :] > pos[:, None]] = -np.inf
+    p = np.exp(s - s.max(axis=2, keepdims=True))
+    ref = np.einsum("hrn,hnd->rhd", p / p.sum(axis=2, keepdims=True), v64)
+    gate = bf(qkv).astype(np.float64).reshape(rows, heads, 2, hd)[:, :, 1]
+    ref = ref * _sigmoid_bf16(gate)
+    dims = mx.AttnDimsC(heads, kv_heads, hd, max_ctx, kv_heads * max_ctx * hd)
+    ws = mx.DeviceArray((mx.lib.mx_attn_workspace_bytes(rows, heads, hd, max_ctx),), np.uint8)
+    dq, dqkv, dsl, dpos, dk, dv = (mx.DeviceArray.from_numpy(np.ascontiguousarray(a))
+                                   for a in (q, qkv, slots, pos, kc, vc))
+    out = mx.DeviceArray((rows, heads, hd), np.uint16)
+    mx.check(mx.lib.mx_attn_decode(dq.ptr, dqkv.ptr, 2 * heads * hd, rows, dsl.ptr, dpos.ptr,
+                                   dk.ptr, dv.ptr, C.byref(dims), 3, ws.ptr, out.ptr, None))
+    g = bf(out.numpy()).astype(np.float64)
+    scale = np.abs(ref).max(axis=2, keepdims=True)
+    assert np.all(np.abs(g - ref) <= 2.0 ** -6 * np.abs(ref) + 2.0 ** -9 * scale)
