@@ -275,6 +275,15 @@ int qmm_chunk_gate_up(const uint16_t* x, const ChunkPlan* plan, int rows, int ex
 int qmm_chunk_down(const uint16_t* h, const ChunkPlan* plan, const uint16_t* scores, int rows,
                    int experts, int top_k, int inter, int shared_inter, const QBank& down,
                    const QWeight& sdown, uint16_t* p, hipStream_t s);
+// the same for depths whose 16 rows fit LDS whole (experts.hip); items: the
+// grid's y extent, hs: elements between h rows
+bool chunk_lds_ok(int k);
+int chunk_gate_up_lds(const uint16_t* x, const ChunkPlan* plan, int items, int top_k,
+                      const QBank& gate, const QBank& up, const QWeight& sgate,
+                      const QWeight& sup, uint16_t* h, hipStream_t s);
+int chunk_down_lds(const uint16_t* h, const ChunkPlan* plan, const uint16_t* scores, int items,
+                   int top_k, int hs, const QBank& down, const QWeight& sdown, uint16_t* p,
+                   hipStream_t s);
 int moe_reduce(const uint16_t* p, int rows, int top_k, int hidden, uint16_t* routed,
                hipStream_t s);
 int moe_hc_epilogue(const uint16_t* routed, const uint16_t* shared, const uint16_t* factor,

@@ -585,6 +585,11 @@ int qmm_down(const uint16_t* h, const MoePlan* plan, const uint16_t* scores, int
   return MX_EUNSUPPORTED;
 }
 
+// Scales and biases that eight-group (16-byte) loads may read.
+bool aligned16(const uint16_t* a, const uint16_t* b) {
+  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
+}
+
 // The 32-row tile forms (4- and 8-bit codes, whole batches of four groups).
 bool chunk_w32_ok(int bits, int k) { return (bits == 4 || bits == 8) && (k >> 6) % 4 == 0; }
 
@@ -593,6 +598,13 @@ int qmm_chunk_gate_up(const uint16_t* x, const ChunkPlan* plan, int rows, int ex
                       const QWeight& sup, uint16_t* h, hipStream_t s) {
   const int hs = gate.n > sgate.n ? gate.n : sgate.n;
   const dim3 grid((hs + 127) / 128, chunk_max_items(rows, experts, top_k));
+  // rows that fit LDS whole: experts.hip, faster at every width and row count
+  // tried (the sublayer's 9 rows 82 -> 76 us, 64 rows 197 -> 167, 512 rows 345 ->
+  // 294; 301 rows at 4 + 5 bits 325 -> 283, 5 + 6 428 -> 367, 8 + 4 377 -> 355)
+  if (chunk_lds_ok(gate.k) && gate.bits == sgate.bits && aligned16(gate.scales, gate.biases) &&
+      aligned16(up.scales, up.biases) && aligned16(sgate.scales, sgate.biases) &&
+      aligned16(sup.scales, sup.biases))
+    return chunk_gate_up_lds(x, plan, int(grid.y), top_k, gate, up, sgate, sup, h, s);
   const bool sx = (gate.k >> 6) % 4 == 0;  // whole batches of four groups
   if (sx && gate.bits == sgate.bits && chunk_w32_ok(gate.bits, gate.k) &&
       chunk_w32_ok(sgate.bits, sgate.k)) {
@@ -627,6 +639,9 @@ int qmm_chunk_down(const uint16_t* h, const ChunkPlan* plan, const uint16_t* sco
                    const QWeight& sdown, uint16_t* p, hipStream_t s) {
   const int hs = inter > shared_inter ? inter : shared_inter;
   const dim3 grid((down.n + 255) / 256, chunk_max_items(rows, experts, top_k));
+  if (chunk_lds_ok(down.k) && chunk_lds_ok(sdown.k) && down.bits == sdown.bits &&
+      aligned16(down.scales, down.biases) && aligned16(sdown.scales, sdown.biases))
+    return chunk_down_lds(h, plan, scores, int(grid.y), top_k, hs, down, sdown, p, s);
   const bool sx = (down.k >> 6) % 4 == 0 && (sdown.k >> 6) % 4 == 0;
   if (sx && down.bits == sdown.bits && chunk_w32_ok(down.bits, down.k) &&
       chunk_w32_ok(sdown.bits, sdown.k)) {
