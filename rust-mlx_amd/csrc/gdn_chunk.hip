@@ -11,8 +11,10 @@
 //   S_t = gamma_t S_0 + sum_{s<=t} (gamma_t / gamma_s) k_s d_s^T
 //   (I + A) D = beta V - (beta gamma K) S_0,  A[t][s] = beta_t (gamma_t/gamma_s) k_t.k_s (s < t)
 //   so D = U - W S_0 with T = (I + A)^-1, U = T (beta V), W = T (beta gamma K);
-//   O = (gamma Q) S_0 + P D,  P[t][s] = (gamma_t/gamma_s) q_t.k_s (s <= t);
-//   S_C = gamma_C S_0 + K'^T D,  K'_s = (gamma_C/gamma_s) k_s.
+//   O = (gamma Q) S_0 + P D = Q' S_0 + P U with Q' = gamma Q - P W,
+//   P[t][s] = (gamma_t/gamma_s) q_t.k_s (s <= t);
+//   S_C = gamma_C S_0 + K'^T D,  K'_s = kappa_s k_s, kappa_s = gamma_C / gamma_s.
+// Q' takes the output off the chain from chunk to chunk, which is D, then S_C.
 // Every product that touches the fp32 state is an fp32 matrix-core product
 // (v_mfma_f32_16x16x4_f32), so the state agrees with the sequential fp32
 // recurrence to rounding; the Gram matrices K K^T and Q K^T of bf16 inputs
@@ -24,6 +26,10 @@
 //    quantities above, written to a workspace in matrix-core operand order.
 //  chunk_scan_kernel (16-column state slices x heads x groups): walks the
 //    chunks in order, carrying its 128 x 16 slice of the state in LDS.
+//
+// An fp32 MFMA step takes one k from each lane quarter; which one is free as
+// long as both operands agree, so a matrix that is read as an operand is laid
+// out for sixteen bytes (four steps) per lane, neighbouring lanes together.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "skinny_core.hpp"
@@ -35,18 +41,28 @@ namespace {
 constexpr int kC = 64;   // tokens per chunk
 constexpr int kD = 128;  // head dim (dk == dv)
 constexpr int kSlice = 16;
-constexpr int kLd = kC + 1;  // padded LDS row
+constexpr int kLd = kC + 1;      // padded LDS row of a C x C matrix
+constexpr int kBLd = kD + 8;     // padded LDS row of a bf16 chunk
+constexpr int kPrepThreads = 512;
+constexpr int kScanThreads = 512;
 
-// Workspace of one (group, head, chunk), in floats.
-constexpr int kWOff = 0;                // W  A-operand order [4 tiles][64 lanes][32]
-constexpr int kQOff = kWOff + kC * kD;  // gamma Q, same order
-constexpr int kKOff = kQOff + kC * kD;  // K'^T A-operand order [8 tiles][64 lanes][16]
-constexpr int kPOff = kKOff + kC * kD;  // P A-operand order [4 tiles][64 lanes][16]
-constexpr int kUOff = kPOff + kC * kC;  // U [64][128]
+// Workspace of one (group, head, chunk), in floats.  A-operand order of an
+// R x 128 matrix: [R / 16 tiles][8][64 lanes][4], element (row, k) in lane
+// 16 (k / 32) + row % 16 at [(k % 32) / 4][k % 4]; of an R x 64 one:
+// [R / 16][4][64][4], element (row, s) in lane 16 (s / 16) + row % 16 at
+// [(s % 16) / 4][s % 4] (K^T, bf16: [8][2][64][8] at [(s % 16) / 8][s % 8]).  U as the B operand of P U: [8 slices][4][64][4],
+// element (s, column) in lane 16 (s / 16) + column % 16 likewise.
+constexpr int kWOff = 0;                // W
+constexpr int kQOff = kWOff + kC * kD;  // Q'
+constexpr int kKOff = kQOff + kC * kD;  // K^T as bf16, then kappa_s = gamma_C / gamma_s
+constexpr int kKappa = kKOff + kC * kD / 2;
+constexpr int kPOff = kKOff + kC * kD;  // P
+constexpr int kUOff = kPOff + kC * kC;  // U
 constexpr int kGOff = kUOff + kC * kD;  // gamma_C
 constexpr int kWsFloats = kGOff + 16;
 
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t uint32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ floatx4_t mfma4(float a, float b, floatx4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -70,39 +86,52 @@ __device__ __forceinline__ void store16(float* Z, int ldz, floatx4_t v, float sc
 }
 
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void chunk_prep_kernel(
+// Eight waves; wave w owns columns 16 w .. + 15 of W, Q' and U for all tokens.
+// W is formed in both orientations from the same operands (products with the
+// operands swapped): transposed it is four consecutive k per lane, as it is
+// stored; untransposed its registers are the A operand of P W.  72 KB of LDS
+// (V takes A's place once T is known): two workgroups per CU.  Bound by the
+// serial inverse and the barriers between its steps; at 32 heads x 32 chunks
+// 52 us, 159 us with four waves, the scales formed per product and every
+// result stored one float per lane.
+__global__ __launch_bounds__(kPrepThreads) void chunk_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const float* __restrict__ g,
     const uint16_t* __restrict__ beta, int hk, int hv, int t, int nchunks, int64_t v_stride,
     float* __restrict__ ws) {
-  __shared__ double Ls[kC];            // inclusive prefix sum of log2 g
-  __shared__ float bs[kC];             // beta
-  __shared__ float Am[kC * kLd];       // K K^T, then A
-  __shared__ float QKm[kC * kLd];      // Q K^T
-  __shared__ float Tm[kC * kLd];       // T = (I + A)^-1
-  __shared__ float tmp[3][16 * 17];    // level products of the blocked inverse
-  __shared__ uint16_t Ks[kC * kD];     // K chunk (bf16)
-  __shared__ uint16_t Vs[kC * kD];     // V chunk (bf16)
+  __shared__ double Ls[kC];                            // inclusive prefix sum of log2 g
+  __shared__ float bs[kC], bg[kC], kp[kC], gm[kC];     // beta, beta gamma, kappa, gamma
+  __shared__ __align__(16) char av[kC * kBLd * 2];     // K K^T, then A; V once T is known
+  __shared__ float QKm[kC * kLd];                      // Q K^T, then P
+  __shared__ float Tm[kC * kLd];                       // T = (I + A)^-1
+  __shared__ float tmp[3][16 * 17];                    // level products of the blocked inverse
+  __shared__ __align__(16) uint16_t Ks[kC * kBLd];     // K chunk
+  static_assert(kC * kLd * 4 <= kC * kBLd * 2, "A fits V's place");
+  float* Am = reinterpret_cast<float*>(av);
+  uint16_t* Vs = reinterpret_cast<uint16_t*>(av);
   const int c = blockIdx.x, h = blockIdx.y, grp = blockIdx.z;
   const int kh = h / (hv / hk);
   const int t0 = c * kC;
   const int len = min(kC, t - t0);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 15, qd = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: whole waves branch
   const size_t row0 = size_t(grp) * t + t0;
   float* out = ws + ((size_t(grp) * hv + h) * nchunks + c) * kWsFloats;
 
-  // K, V chunk into LDS (rows past len are zero); 16-byte units
-  for (int u = tid; u < kC * kD / 8; u += 256) {
-    const int r = u / (kD / 8), cu = u - r * (kD / 8);
+  // K chunk into LDS, V chunk into registers (rows past len are zero)
+  uint4 vreg[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int u = tid + i * kPrepThreads;  // 16-byte piece
+    const int r = u >> 4, cu = u & 15;
     const bool ok = r < len;
     const size_t rr = row0 + (ok ? r : 0);
     uint4 kv = *reinterpret_cast<const uint4*>(k + (rr * hk + kh) * kD + cu * 8);
-    uint4 vv = *reinterpret_cast<const uint4*>(v + rr * v_stride + h * kD + cu * 8);
-    if (!ok) kv = vv = make_uint4(0u, 0u, 0u, 0u);
-    *reinterpret_cast<uint4*>(Ks + r * kD + cu * 8) = kv;
-    *reinterpret_cast<uint4*>(Vs + r * kD + cu * 8) = vv;
+    vreg[i] = *reinterpret_cast<const uint4*>(v + rr * v_stride + h * kD + cu * 8);
+    if (!ok) kv = vreg[i] = make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(Ks + r * kBLd + cu * 8) = kv;
   }
-  // log2 g prefix (fp64, wave 0) and beta
+  // log2 g prefix (fp64, wave 0), beta and the scales made of them
   if (tid < kC) {
     const bool ok = tid < len;
     const float gv = ok ? g[(row0 + tid) * hv + h] : 1.0f;
@@ -113,53 +142,56 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
       const double n = __shfl_up(l, o, 64);
       if (lane >= o) l += n;
     }
+    const double lc = __shfl(l, kC - 1, 64);
+    const float gt = __builtin_amdgcn_exp2f(float(l));
     Ls[tid] = l;
     bs[tid] = bv;
+    gm[tid] = gt;
+    bg[tid] = bv * gt;
+    kp[tid] = __builtin_amdgcn_exp2f(float(lc - l));
+    if (tid == kC - 1) out[kGOff] = gt;
   }
-  // Gram matrices on the bf16 matrix cores (exact products, fp32 sums):
-  // wave w computes row tile w of K K^T and of Q K^T
-  {
-    const int rt = wave;
-    const int ra = min(t0 + 16 * rt + j, t - 1) - t0;  // clamped token of this lane's A row
+  // this wave's Gram rows: K (waves 0..3, from LDS) or Q (waves 4..7)
+  const int rt = wave & 3;
+  uint4 ga[kD / 32];
+  if (wave >= 4) {
     const bool rok = 16 * rt + j < len;
-    sk::floatx4_t gk[4], gq[4];
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct) gk[ct] = gq[ct] = sk::floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint16_t* qr = q + ((row0 + (rok ? 16 * rt + j : 0)) * hk + kh) * kD + 8 * qd;
 #pragma unroll
     for (int kk = 0; kk < kD / 32; ++kk) {
-      const int d0 = 32 * kk + 8 * qd;
-      uint4 ak = *reinterpret_cast<const uint4*>(k + ((row0 + ra) * hk + kh) * kD + d0);
-      uint4 aq = *reinterpret_cast<const uint4*>(q + ((row0 + ra) * hk + kh) * kD + d0);
-      if (!rok) ak = aq = make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const int cb = min(t0 + 16 * ct + j, t - 1) - t0;
-        uint4 bk = *reinterpret_cast<const uint4*>(k + ((row0 + cb) * hk + kh) * kD + d0);
-        if (16 * ct + j >= len) bk = make_uint4(0u, 0u, 0u, 0u);
-        gk[ct] = sk::mfma(ak, bk, gk[ct]);
-        gq[ct] = sk::mfma(aq, bk, gq[ct]);
-      }
+      ga[kk] = *reinterpret_cast<const uint4*>(qr + 32 * kk);
+      if (!rok) ga[kk] = make_uint4(0u, 0u, 0u, 0u);
     }
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        Am[(16 * rt + 4 * qd + r) * kLd + 16 * ct + j] = gk[ct][r];
-        QKm[(16 * rt + 4 * qd + r) * kLd + 16 * ct + j] = gq[ct][r];
-      }
   }
   __syncthreads();
-  // A (strictly lower) and P (lower incl. diagonal) with the decay ratios
-  for (int e = tid; e < kC * kC; e += 256) {
-    const int tr = e >> 6, sc = e & 63;
-    const float ratio = sc <= tr ? __builtin_amdgcn_exp2f(float(Ls[tr] - Ls[sc])) : 0.0f;
-    Am[tr * kLd + sc] = sc < tr ? bs[tr] * ratio * Am[tr * kLd + sc] : 0.0f;
-    QKm[tr * kLd + sc] = ratio * QKm[tr * kLd + sc];
+  {
+    if (wave < 4)
+#pragma unroll
+      for (int kk = 0; kk < kD / 32; ++kk)
+        ga[kk] = *reinterpret_cast<const uint4*>(Ks + (16 * rt + j) * kBLd + 32 * kk + 8 * qd);
+    float* dst = wave < 4 ? Am : QKm;
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) {
+      sk::floatx4_t gr = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kk = 0; kk < kD / 32; ++kk)
+        gr = sk::mfma(ga[kk],
+                      *reinterpret_cast<const uint4*>(Ks + (16 * ct + j) * kBLd + 32 * kk + 8 * qd),
+                      gr);
+      // A (strictly lower) and P (lower incl. diagonal) with the decay ratios
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tr = 16 * rt + 4 * qd + r, sc = 16 * ct + j;
+        const float ratio = sc <= tr ? __builtin_amdgcn_exp2f(float(Ls[tr] - Ls[sc])) : 0.0f;
+        dst[tr * kLd + sc] =
+            wave >= 4 ? ratio * gr[r] : sc < tr ? bs[tr] * ratio * gr[r] : 0.0f;
+      }
+    }
   }
   __syncthreads();
   // T = (I + A)^-1, blocked 4 x 4 over 16 x 16 blocks.
-  // Diagonal blocks: wave w, lane j < 16 owns column j of block w.
-  if (j == lane) {  // lanes 0..15 of every wave
+  // Diagonal blocks: wave w < 4, lane j < 16 owns column j of block w.
+  if (wave < 4 && j == lane) {
     const int b0 = 16 * wave;
     float col[16];
 #pragma unroll
@@ -172,13 +204,25 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
 #pragma unroll
     for (int r = 0; r < 16; ++r) Tm[(b0 + r) * kLd + b0 + j] = col[r];
   }
-  // zero the strictly upper blocks
-  for (int e = tid; e < kC * kC; e += 256) {
-    const int tr = e >> 6, sc = e & 63;
-    if ((sc >> 4) > (tr >> 4)) Tm[tr * kLd + sc] = 0.0f;
+  if (wave >= 4) {  // meanwhile: K^T, kappa and P, eight or four s per lane
+    for (int f = tid - 256; f < kC * kD / 8; f += 256) {
+      const int l = f & 63, d = 16 * (f >> 7) + (l & 15), s = 16 * (l >> 4) + 8 * ((f >> 6) & 1);
+      uint32_t o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[i] = uint32_t(Ks[(s + 2 * i) * kBLd + d]) | (uint32_t(Ks[(s + 2 * i + 1) * kBLd + d]) << 16);
+      reinterpret_cast<uint4*>(out + kKOff)[f] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    if (tid - 256 < kC) out[kKappa + tid - 256] = kp[tid - 256];
+    for (int f = tid - 256; f < kC * kC / 4; f += 256) {
+      const int l = f & 63, i4 = (f >> 6) & 3, tr = 16 * (f >> 8) + (l & 15), s = 16 * (l >> 4) + 4 * i4;
+      const float* p = QKm + tr * kLd + s;
+      reinterpret_cast<float4*>(out + kPOff)[f] = make_float4(p[0], p[1], p[2], p[3]);
+    }
   }
   __syncthreads();
   // off-diagonal blocks by distance: T_ij = -T_ii sum_{m=j}^{i-1} A_im T_mj
+  // (blocks above the diagonal are never read)
   for (int dist = 1; dist < 4; ++dist) {
     const int bi = wave + dist, bj = wave;  // waves 0 .. 3 - dist
     const bool act = bi < 4;
@@ -187,198 +231,234 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(
       for (int m = bj; m < bi; ++m)
         acc = mm16(Am + (16 * bi) * kLd + 16 * m, kLd, Tm + (16 * m) * kLd + 16 * bj, kLd, acc);
       store16(tmp[wave], 17, acc, 1.0f);
-    }
-    __syncthreads();
-    if (act) {
-      floatx4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+      __builtin_amdgcn_wave_barrier();
+      acc = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
       acc = mm16(Tm + (16 * bi) * kLd + 16 * bi, kLd, tmp[wave], 17, acc);
       store16(Tm + (16 * bi) * kLd + 16 * bj, kLd, acc, -1.0f);
     }
     __syncthreads();
   }
-  // W = T (beta gamma K), U = T (beta V): 4 row tiles x 8 column tiles each;
-  // wave w takes row tile w.  B values formed on the fly from LDS.
-  {
-    const int rt = wave;
-    float* wop = out + kWOff;
-    float* uo = out + kUOff;
-    for (int ct = 0; ct < kD / 16; ++ct) {
-      floatx4_t aw = {0.0f, 0.0f, 0.0f, 0.0f}, au = aw;
-#pragma unroll 4
-      for (int kk = 0; kk < kC / 4; ++kk) {
-        const int s = 4 * kk + qd;
-        const float a = Tm[(16 * rt + j) * kLd + s];
-        const float bsc = bs[s];
-        const float gs = __builtin_amdgcn_exp2f(float(Ls[s]));
-        aw = mfma4(a, bsc * gs * bf16_to_f32(Ks[s * kD + 16 * ct + j]), aw);
-        au = mfma4(a, bsc * bf16_to_f32(Vs[s * kD + 16 * ct + j]), au);
-      }
-      // W in A-operand order: tile rt, lane (row j', k-slot q'), index kk'
-      // element W[16 rt + rr][d] with d = 16 ct + j -> kk' = d / 4, q' = d % 4
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int rr = 4 * qd + r, d = 16 * ct + j;
-        const int l2 = (d & 3) * 16 + rr;
-        wop[(rt * 64 + l2) * 32 + (d >> 2)] = aw[r];
-        uo[(16 * rt + rr) * kD + d] = au[r];
-      }
-    }
+  for (int i = 0; i < 2; ++i) {
+    const int u = tid + i * kPrepThreads;
+    *reinterpret_cast<uint4*>(Vs + (u >> 4) * kBLd + (u & 15) * 8) = vreg[i];
   }
-  // gamma Q (A-operand order like W), K'^T (A operand rows d, k = s), P
-  {
-    const double lc = Ls[kC - 1];
-    float* qop = out + kQOff;
-    float* kop = out + kKOff;
-    float* pop = out + kPOff;
-    for (int e = tid; e < kC * kD; e += 256) {
-      const int tr = e >> 7, d = e & 127;
-      const bool ok = tr < len;
-      const size_t rr = row0 + (ok ? tr : 0);
-      const float qv = ok ? bf16_to_f32(q[(rr * hk + kh) * kD + d]) : 0.0f;
-      const float gt = __builtin_amdgcn_exp2f(float(Ls[tr]));
-      // gamma Q: tile tr / 16, lane (d % 4) * 16 + tr % 16, index d / 4
-      qop[((tr >> 4) * 64 + (d & 3) * 16 + (tr & 15)) * 32 + (d >> 2)] = gt * qv;
-      // K'^T [d][s = tr]: tile d / 16, lane (s % 4) * 16 + d % 16, index s / 4
-      const float kv = bf16_to_f32(Ks[tr * kD + d]) * __builtin_amdgcn_exp2f(float(lc - Ls[tr]));
-      kop[((d >> 4) * 64 + (tr & 3) * 16 + (d & 15)) * 16 + (tr >> 2)] = kv;
+  __syncthreads();
+  // columns 16 wave + j of K and V as operands: k-step i takes s = 4 i + qd
+  float kc[16], vc[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int s = 4 * i + qd;
+    kc[i] = bf16_to_f32(Ks[s * kBLd + 16 * wave + j]) * bg[s];
+    vc[i] = bf16_to_f32(Vs[s * kBLd + 16 * wave + j]) * bs[s];
+  }
+  floatx4_t wn[4];  // W rows 16 tt + 4 qd + r, column 16 wave + j
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt) {
+    floatx4_t wt = {0.0f, 0.0f, 0.0f, 0.0f}, un = wt;
+    wn[tt] = wt;
+#pragma unroll
+    for (int i = 0; i < 4 * (tt + 1); ++i) {
+      const float a = Tm[(16 * tt + j) * kLd + 4 * i + qd];
+      wt = mfma4(kc[i], a, wt);
+      wn[tt] = mfma4(a, kc[i], wn[tt]);
+      un = mfma4(a, vc[i], un);
     }
-    for (int e = tid; e < kC * kC; e += 256) {
-      const int tr = e >> 6, sc = e & 63;
-      pop[((tr >> 4) * 64 + (sc & 3) * 16 + (tr & 15)) * 16 + (sc >> 2)] = QKm[tr * kLd + sc];
-    }
-    if (tid == 0) out[kGOff] = __builtin_amdgcn_exp2f(float(lc));
+    // W^T tile: lane token 16 tt + j, k = 16 wave + 4 qd ..
+    reinterpret_cast<floatx4_t*>(out + kWOff)[(tt * 8 + 4 * (wave & 1) + qd) * 64 +
+                                              (wave >> 1) * 16 + j] = wt;
+    // U tile: tokens 16 tt + 4 qd .., column 16 wave + j
+    reinterpret_cast<floatx4_t*>(out + kUOff)[(wave * 4 + qd) * 64 + tt * 16 + j] = un;
+  }
+  // Q'^T tile: lane token 16 tt + j, k = 16 wave + 4 qd ..; k-step (b, r) takes
+  // s = 16 b + 4 qd + r
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt) {
+    floatx4_t pw = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b <= tt; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        pw = mfma4(wn[b][r], QKm[(16 * tt + j) * kLd + 16 * b + 4 * qd + r], pw);
+    const int tr = 16 * tt + j;
+    const bool ok = tr < len;
+    const uint2 qv = *reinterpret_cast<const uint2*>(
+        q + ((row0 + (ok ? tr : 0)) * hk + kh) * kD + 16 * wave + 4 * qd);
+    const float gt = ok ? gm[tr] : 0.0f;
+    floatx4_t qo;
+    qo[0] = fmaf_(gt, u2f(qv.x << 16), -pw[0]);
+    qo[1] = fmaf_(gt, u2f(qv.x & 0xffff0000u), -pw[1]);
+    qo[2] = fmaf_(gt, u2f(qv.y << 16), -pw[2]);
+    qo[3] = fmaf_(gt, u2f(qv.y & 0xffff0000u), -pw[3]);
+    reinterpret_cast<floatx4_t*>(out + kQOff)[(tt * 8 + 4 * (wave & 1) + qd) * 64 +
+                                              (wave >> 1) * 16 + j] = qo;
   }
 }
 
 // ---------------------------------------------------------------------------
-// One 16-column slice of one head's state, chunk after chunk.  Wave w owns
-// output row tile w (tokens 16 w ..) and state row tiles 2 w, 2 w + 1.
-__global__ __launch_bounds__(256) void chunk_scan_kernel(const float* __restrict__ ws, int hv,
-                                                         int t, int nchunks,
-                                                         const int32_t* __restrict__ slots,
-                                                         float* __restrict__ state,
-                                                         uint16_t* __restrict__ y) {
-  __shared__ float Sl[kD * 17];  // state slice [d][16]
-  __shared__ float Dl[kC * 17];  // D of the chunk [s][16]
-  const int slice = blockIdx.x, h = blockIdx.y, grp = blockIdx.z;
+// One 16-column slice of one head's state, chunk after chunk.  Waves 0..3
+// carry the chain (wave w: rows 16 w .. of D, then state row tiles 2 w and
+// 2 w + 1), waves 4..7 the outputs (wave 4 + w: tokens 16 w ..), which only
+// read the state that enters the chunk.  State and D lie in LDS by column, so
+// an operand is sixteen bytes per lane; both copies of the state alternate, so
+// a chunk takes two barriers.  Operands are requested a chunk ahead (they do
+// not depend on the state).  At 32 heads x 32 chunks 114 us, 3.6 us a chunk,
+// 213 us with one wave per SIMD doing both, the output after D.  Bound by the
+// workspace's way from L2 (every slice reads 98 KB a chunk: 89 us with chunk
+// 0's operands throughout; fp32 K'^T and all of P cost 14 us, slices of a head
+// on different XCDs 16 us) and by the chain's two barriers and 64 fp32 MFMAs.
+__global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(
+    const float* __restrict__ ws, int hv, int t, int nchunks, const int32_t* __restrict__ slots,
+    float* __restrict__ state, uint16_t* __restrict__ y) {
+  constexpr int kSLd = kD + 4, kDLd = kC + 4;
+  __shared__ __align__(16) float Sl[2][kSlice * kSLd];  // state slice [column][d]
+  __shared__ __align__(16) float Dl[kSlice * kDLd];     // D of the chunk [column][s]
+  // the eight slices of a head read the same workspace: on one XCD (workgroup
+  // ids mod 8) they share its L2, when the heads divide among the XCDs
+  static_assert(kD / kSlice == 8, "eight slices");
+  const int id = blockIdx.x + 8 * (blockIdx.y + gridDim.y * blockIdx.z);
+  const bool even = (gridDim.y * gridDim.z) % 8 == 0;
+  const int slice = even ? (id >> 3) & 7 : id & 7;
+  const int head = even ? (id >> 6) * 8 + (id & 7) : id >> 3;  // of all groups
+  const int h = head % hv, grp = head / hv;
   const int i0 = slice * kSlice;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 15, qd = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: whole waves branch
+  const int w = wave & 3;
   float* sp = state + (size_t(slots[grp]) * hv + h) * kD * kD + i0;
-  for (int e = tid; e < kD * kSlice; e += 256) {
-    const int d = e >> 4, i = e & 15;
-    Sl[d * 17 + i] = sp[size_t(d) * kD + i];
-  }
-  __syncthreads();
-  // a chunk's workspace operands of this lane; the next chunk's are
-  // requested before this chunk's work (they do not depend on the state)
-  struct ChunkOps {
-    float4 w[8], q[8], p[4], k[2][4];
-    float u[4];
-    float gc;
-  };
-  auto load_ops = [&](int c, ChunkOps& o) {
-    const float* in = ws + ((size_t(grp) * hv + h) * nchunks + c) * kWsFloats;
-    const float4* wrow = reinterpret_cast<const float4*>(in + kWOff + (wave * 64 + lane) * 32);
-    const float4* qrow = reinterpret_cast<const float4*>(in + kQOff + (wave * 64 + lane) * 32);
+  for (int e = tid; e < kD * kSlice; e += kScanThreads)
+    Sl[0][(e & 15) * kSLd + (e >> 4)] = sp[size_t(e >> 4) * kD + (e & 15)];
+  const float* in = ws + (size_t(grp) * hv + h) * nchunks * kWsFloats;
+  const floatx4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (wave < 4) {
+    struct Ops {
+      floatx4_t w[8], u, kappa;
+      uint32x4_t k[2][2];
+      float gc;
+    };
+    auto load = [&](int c, Ops& o) __attribute__((always_inline)) {
+      const floatx4_t* p = reinterpret_cast<const floatx4_t*>(in + size_t(c) * kWsFloats);
 #pragma unroll
-    for (int k4 = 0; k4 < 8; ++k4) {
-      o.w[k4] = wrow[k4];
-      o.q[k4] = qrow[k4];
-    }
-    const float4* prow = reinterpret_cast<const float4*>(in + kPOff + (wave * 64 + lane) * 16);
+      for (int i = 0; i < 8; ++i) o.w[i] = p[kWOff / 4 + (w * 8 + i) * 64 + lane];
 #pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4) o.p[k4] = k4 <= wave ? prow[k4] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float4* krow =
-          reinterpret_cast<const float4*>(in + kKOff + ((2 * wave + u) * 64 + lane) * 16);
-#pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4) o.k[u][k4] = krow[k4];
-    }
-    const float* uo = in + kUOff;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o.u[r] = uo[(16 * wave + 4 * qd + r) * kD + i0 + j];
-    o.gc = in[kGOff];
-  };
-  ChunkOps cur, nxt;
-  load_ops(0, cur);
-  for (int c = 0; c < nchunks; ++c) {
-    if (c + 1 < nchunks) load_ops(c + 1, nxt);  // in flight during this chunk
-    const int t0 = c * kC;
-    const int len = min(kC, t - t0);
-    // D = U - W S and the first part of O = (gamma Q) S, row tile `wave`
-    floatx4_t dacc = {0.0f, 0.0f, 0.0f, 0.0f}, oacc = dacc;
-#pragma unroll
-    for (int k4 = 0; k4 < 8; ++k4) {
-      const float4 wv = cur.w[k4], qv = cur.q[k4];
-      const float wa[4] = {wv.x, wv.y, wv.z, wv.w}, qa[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int kk = 4 * k4 + e;
-        const float sb = Sl[(4 * kk + qd) * 17 + j];
-        dacc = mfma4(wa[e], sb, dacc);
-        oacc = mfma4(qa[e], sb, oacc);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tr = 16 * wave + 4 * qd + r;
-      Dl[tr * 17 + j] = cur.u[r] - dacc[r];
-    }
-    const float gc = cur.gc;
+        for (int i = 0; i < 2; ++i)
+          o.k[u][i] = reinterpret_cast<const uint32x4_t*>(
+              p)[kKOff / 4 + ((2 * w + u) * 2 + i) * 64 + lane];
+      o.kappa = p[kKappa / 4 + 4 * w + qd];
+      o.u = p[kUOff / 4 + (slice * 4 + qd) * 64 + w * 16 + j];  // tokens 16 w + 4 qd ..
+      o.gc = in[size_t(c) * kWsFloats + kGOff];
+    };
+    Ops cur, nxt;
+    load(0, cur);
     __syncthreads();
-    // O += P D (P lower triangular: k-steps up to the tile's diagonal)
+    for (int c = 0; c < nchunks; ++c) {
+      load(min(c + 1, nchunks - 1), nxt);
+      const float* S = Sl[c & 1];
+      floatx4_t d0 = zero, d1 = zero;  // two chains: even and odd pieces of k
 #pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4) {
-      if (k4 > wave) break;  // uniform per wave
-      const float4 pv = cur.p[k4];
-      const float pa[4] = {pv.x, pv.y, pv.z, pv.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int kk = 4 * k4 + e;
-        oacc = mfma4(pa[e], Dl[(4 * kk + qd) * 17 + j], oacc);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tr = 16 * wave + 4 * qd + r;
-      if (tr < len)
-        y[((size_t(grp) * t + t0 + tr) * hv + h) * kD + i0 + j] = f32_to_bf16(oacc[r]);
-    }
-    // S_new = gamma_C S + K'^T D for state row tiles 2 wave, 2 wave + 1
-    floatx4_t sacc[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int dt = 2 * wave + u;
-      floatx4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4) {
-        const float4 kv = cur.k[u][k4];
-        const float ka[4] = {kv.x, kv.y, kv.z, kv.w};
+      for (int i = 0; i < 8; i += 2) {
+        const floatx4_t s0 = *reinterpret_cast<const floatx4_t*>(S + j * kSLd + 32 * qd + 4 * i);
+        const floatx4_t s1 = *reinterpret_cast<const floatx4_t*>(S + j * kSLd + 32 * qd + 4 * i + 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int kk = 4 * k4 + e;
-          acc = mfma4(ka[e], Dl[(4 * kk + qd) * 17 + j], acc);
+          d0 = mfma4(cur.w[i][e], s0[e], d0);
+          d1 = mfma4(cur.w[i + 1][e], s1[e], d1);
         }
       }
+      // kappa D: K'^T D is K^T (kappa D), with K as it came
+      floatx4_t dk = cur.u - (d0 + d1);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = fmaf_(gc, Sl[(16 * dt + 4 * qd + r) * 17 + j], acc[r]);
-      sacc[u] = acc;
+      for (int r = 0; r < 4; ++r) dk[r] = dk[r] * cur.kappa[r];
+      *reinterpret_cast<floatx4_t*>(Dl + j * kDLd + 16 * w + 4 * qd) = dk;
+      __syncthreads();  // D is whole
+      floatx4_t a[2] = {zero, zero};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const floatx4_t dv = *reinterpret_cast<const floatx4_t*>(Dl + j * kDLd + 16 * qd + 4 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const uint32_t kw = cur.k[u][i >> 1][2 * (i & 1) + (e >> 1)];
+            a[u] = mfma4(u2f((e & 1) ? (kw & 0xffff0000u) : (kw << 16)), dv[e], a[u]);
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int at = j * kSLd + 16 * (2 * w + u) + 4 * qd;
+        const floatx4_t old = *reinterpret_cast<const floatx4_t*>(S + at);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[u][r] = fmaf_(cur.gc, old[r], a[u][r]);
+        *reinterpret_cast<floatx4_t*>(Sl[(c + 1) & 1] + at) = a[u];
+      }
+      __syncthreads();  // the next state is whole
+      cur = nxt;
     }
-    __syncthreads();  // every read of Sl and Dl for this chunk is done
+  } else {
+    struct Ops {
+      floatx4_t q[8], p[4], u[4];
+    };
+    auto load = [&](int c, Ops& o) __attribute__((always_inline)) {
+      const floatx4_t* p = reinterpret_cast<const floatx4_t*>(in + size_t(c) * kWsFloats);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int dt = 2 * wave + u;
+      for (int i = 0; i < 8; ++i) o.q[i] = p[kQOff / 4 + (w * 8 + i) * 64 + lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) Sl[(16 * dt + 4 * qd + r) * 17 + j] = sacc[u][r];
-    }
+      for (int i = 0; i < 4; ++i) {
+        // quarters past the tile's tokens multiply nothing (P is lower triangular)
+        o.p[i] = o.u[i] = zero;
+        if (qd <= w) {
+          o.p[i] = p[kPOff / 4 + (w * 4 + i) * 64 + lane];
+          o.u[i] = p[kUOff / 4 + (slice * 4 + i) * 64 + lane];
+        }
+      }
+    };
+    Ops cur, nxt;
+    load(0, cur);
     __syncthreads();
-    cur = nxt;
+    for (int c = 0; c < nchunks; ++c) {
+      load(min(c + 1, nchunks - 1), nxt);
+      const float* S = Sl[c & 1];
+      floatx4_t o0 = zero, o1 = zero;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (i & 1)
+            o1 = mfma4(cur.p[i][e], cur.u[i][e], o1);
+          else
+            o0 = mfma4(cur.p[i][e], cur.u[i][e], o0);
+        }
+      // half of the state's products before the barrier on D, half after it
+      // (the chain has the matrix cores to itself for as long either way)
+      auto half = [&](int i) __attribute__((always_inline)) {
+        const floatx4_t s0 = *reinterpret_cast<const floatx4_t*>(S + j * kSLd + 32 * qd + 4 * i);
+        const floatx4_t s1 = *reinterpret_cast<const floatx4_t*>(S + j * kSLd + 32 * qd + 4 * i + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          o0 = mfma4(cur.q[i][e], s0[e], o0);
+          o1 = mfma4(cur.q[i + 1][e], s1[e], o1);
+        }
+      };
+      half(0);
+      __syncthreads();
+      half(2);
+      half(4);
+      half(6);
+      const floatx4_t o = o0 + o1;
+      const int t0 = c * kC;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tr = t0 + 16 * w + 4 * qd + r;
+        if (tr < t) y[((size_t(grp) * t + tr) * hv + h) * kD + i0 + j] = f32_to_bf16(o[r]);
+      }
+      __syncthreads();
+      cur = nxt;
+    }
   }
-  for (int e = tid; e < kD * kSlice; e += 256) {
-    const int d = e >> 4, i = e & 15;
-    sp[size_t(d) * kD + i] = Sl[d * 17 + i];
-  }
+  for (int e = tid; e < kD * kSlice; e += kScanThreads)
+    sp[size_t(e >> 4) * kD + (e & 15)] = Sl[nchunks & 1][(e & 15) * kSLd + (e >> 4)];
 }
 
 }  // namespace
@@ -396,9 +476,9 @@ int gdn_prefill_chunked(const uint16_t* q, const uint16_t* k, const uint16_t* v,
   if (groups <= 0 || t <= 0) return MX_OK;
   const int nchunks = (t + kC - 1) / kC;
   if (v_stride <= 0) v_stride = int64_t(d.hv) * kD;
-  hipLaunchKernelGGL(chunk_prep_kernel, dim3(nchunks, d.hv, groups), dim3(256), 0, s, q, k, v, g,
+  hipLaunchKernelGGL(chunk_prep_kernel, dim3(nchunks, d.hv, groups), dim3(kPrepThreads), 0, s, q, k, v, g,
                      beta, d.hk, d.hv, t, nchunks, v_stride, workspace);
-  hipLaunchKernelGGL(chunk_scan_kernel, dim3(kD / kSlice, d.hv, groups), dim3(256), 0, s,
+  hipLaunchKernelGGL(chunk_scan_kernel, dim3(kD / kSlice, d.hv, groups), dim3(kScanThreads), 0, s,
                      workspace, d.hv, t, nchunks, slots, state, y);
   return hipGetLastError() == hipSuccess ? MX_OK : MX_EHIP;
 }
