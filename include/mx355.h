@@ -441,7 +441,7 @@ mx_status mx_gemv_bf16(const uint16_t* w, int32_t n, int32_t k, const uint16_t* 
  * tolerance) instead of the fixed-order kernel that the CPU oracle restates.
  * flags bit 1: the matrix-core prefill form (within the same tolerance) for
  * the rows of one slot's prompt chunk: blocks of 8 * 16 / (heads / kv_heads)
- * rows share each 64-key tile, with partials per 256-key split; every row
+ * rows share each 64-key tile, with partials per split of the keys; every row
  * must name the same slot; needs head_dim 128 or 256 and 2, 4 or 8 q heads
  * per kv head (MX_EUNSUPPORTED otherwise).
  * workspace: mx_attn_workspace_bytes(rows, heads, head_dim, max_ctx) bytes.
