@@ -95,6 +95,7 @@ enum : int {
   kSrcPlaneLds = 3,  // the producer's plane copied once per workgroup into LDS
   kSrcBlockLds = 4,  // one four-row block of the plane copied into LDS (blockIdx.y)
   kSrcBlockPlane = 5,  // one four-row block of the plane read in place by each wave
+  kSrcReady = 6,       // in LDS already (no copy, no barrier, KS = 1 only)
 };
 
 template <int BITS>
@@ -398,7 +399,7 @@ __device__ __forceinline__ void xq_tiles(const uint32_t* __restrict__ crow,
       yt[i] = float(total);
     }
   }
-  __syncthreads();
+  if constexpr (SRC != kSrcReady) __syncthreads();
 }
 
 // Dense projections (modes of ProjEpilogue).  Workgroup tg covers rows
@@ -459,6 +460,56 @@ __global__ __launch_bounds__(64 * T * KS) void xq_dense_kernel(QWeight w,
                                       XRows{x, x_stride}, plane, lds, yt,
                                       [&] { fin.prefetch(e); }, rm);
   fin.finish(yt, e, tg, M, n);
+}
+
+// Plain projections of long matrices: a workgroup makes its operands once and
+// its waves then stream 16-row tiles over the whole depth, one after another
+// and without barriers (the sums in slice order, so the same values as
+// xq_dense_kernel gives).  That kernel digitises the activation rows again for
+// every 64 weight rows and meets three times for each.  Bound by the weight
+// stream: 8 rows x 151936 x 2048, 8 bits 66.3 us (5.0 TB/s), 109.8 before; 4
+// bits 47.0 (87.4), 6 bits 62.6 (107.4).
+constexpr int kLongWaves = 8, kLongPerCu = 2;  // 69 KB of LDS, 94-122 registers
+// More rows than one round of xq_dense_kernel's 64-row workgroups (one fits a
+// CU) covers.  16000 rows of 4 bits: 8.4 / 10.3 us there (1 / 8 activation
+// rows), 11.2 / 15.0 here; 20000: 13.4 / 17.7 there, 11.4 / 15.4 here (6 bits
+// 15.8 / 21.2 and 14.5 / 18.5, 8 bits 15.3 / 20.3 and 11.6 / 15.6).
+constexpr int kLongRows = 256 * 64;
+
+template <int BITS, int SPW, bool RM>
+__global__ __launch_bounds__(64 * kLongWaves) __attribute__((amdgpu_waves_per_eu(4)))
+void xq_long_kernel(QWeight w, const uint16_t* __restrict__ x, int64_t x_stride, int M,
+                    ProjEpilogue e) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ float yt[8 * 16 * kLongWaves];
+  constexpr int NC = 16 * kLongWaves;
+  const int lane = threadIdx.x & 63, j = lane & 15, kb = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = w.n, G = w.k / xq::kGroup, tiles = (n + 15) / 16;
+  xq::stage<64 * kLongWaves>(lds, XRows{x, x_stride}, M, 0, G);
+  const size_t words = size_t(w.k) * BITS / 32;
+  const bool sbv = tiles_sbv<BITS, SPW>(w);
+  // workgroups before waves: a last round that is not full spreads over the CUs
+  for (int tile = wave * gridDim.x + blockIdx.x; tile < tiles; tile += kLongWaves * gridDim.x) {
+    const int row = min(16 * tile + j, n - 1);
+    RmRows rm;
+    if constexpr (RM) {
+      const int lrow = min(16 * tile + (lane >> 2), n - 1);
+      rm.codes = w.codes + lrow * words;
+      rm.scales = w.scales + size_t(lrow) * G;
+      rm.biases = w.biases + size_t(lrow) * G;
+    }
+    xq_tiles<BITS, kLongWaves, 1, SPW, kSrcReady, RM>(
+        w.codes + row * words, w.scales + size_t(row) * G, w.biases + size_t(row) * G, sbv, w.k, M,
+        M > 4 ? 3 : 1, XRows{x, x_stride}, nullptr, lds, yt, [] {}, rm);
+    if (16 * tile + j < n)  // this lane's own two sums
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int m = 4 * b + kb;
+        if (m < M)
+          e.y[size_t(m) * e.y_stride + 16 * tile + j] = f32_to_bf16(yt[m * NC + 16 * wave + j]);
+      }
+  }
 }
 
 // Activation rows of an expert plan entry: member m is route (row, slot) at
@@ -974,6 +1025,27 @@ int launch_xq(const QWeight& w, const uint16_t* x, int64_t xs, int m, const char
   return hipGetLastError() == hipSuccess ? MX_OK : MX_EHIP;
 }
 
+template <int BITS, int SPW>
+int launch_long(const QWeight& w, const uint16_t* x, int64_t xs, int m, const ProjEpilogue& e,
+                hipStream_t s) {
+  const int G = w.k / xq::kGroup, tiles = (w.n + 15) / 16;
+  constexpr int B = tile_batch<BITS, SPW>();
+  // row-major weight reads as in launch_xq
+  const bool rm = B % 2 == 0 && G == 2 * SPW &&
+                  (BITS == 5 || BITS == 6 ||
+                   ((reinterpret_cast<uintptr_t>(w.codes) & 15) == 0 &&
+                    (size_t(w.k) * BITS / 8) % 16 == 0)) &&
+                  xq::sb_vector_ok<B>(w.scales, w.biases, G);
+  constexpr bool kRm = B % 2 == 0;
+  auto fn = rm ? xq_long_kernel<BITS, SPW, kRm> : xq_long_kernel<BITS, SPW, false>;
+  const int lb = tiles_lds(G, kLongWaves, 1, kSrcStage);
+  MX_TRY_RC(raise_lds(fn, lb));
+  const int full = 256 * kLongPerCu, need = (tiles + kLongWaves - 1) / kLongWaves;
+  hipLaunchKernelGGL(fn, dim3(need < full ? need : full), dim3(64 * kLongWaves), lb, s, w, x, xs, m,
+                     e);
+  return hipGetLastError() == hipSuccess ? MX_OK : MX_EHIP;
+}
+
 // Slices of two groups: S = 1..4 slices run in one wave (four tiles per
 // workgroup); deeper rows split their slices over KS waves of one tile (16
 // waves at K = 2048 for up to 2048 rows, so short matrices still fill the
@@ -998,6 +1070,8 @@ int xq_shape(const QWeight& w, const uint16_t* x, int64_t xs, int m, const char*
       MX_XQ(4, 2, 4, kSrcStage);
     }
     if (S == 16) {
+      if constexpr (MODE == kPlain && BITS != 5)  // (5 bits: 136 bytes of spills)
+        if (!plane && w.n > kLongRows) return launch_long<BITS, 16>(w, x, xs, m, e, s);
       if (w.n > 2048) {
         if (plane) MX_XQ(4, 4, 4, kSrcPlaneLds);
         MX_XQ(4, 4, 4, kSrcStage);
