@@ -11,7 +11,7 @@
 // many vector instructions: 124 us against 91 us at 512 x 12352 x 2048 in one
 // and the same 128-row form).
 //
-// Two forms (launch_gemm chooses by an estimate of their times):
+// Two forms (gemm_plan chooses by an estimate of their times):
 //  gemm_tile_kernel  a workgroup computes 64 weight rows x 32 UW activation
 //    rows from LDS, one group at a time.
 //  gemm_deep_kernel  few output tiles: every wave of a workgroup takes the
@@ -21,6 +21,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "gemm_plan.hpp"
 #include "kernels.hpp"
 #include "qmm_core.hpp"
 
@@ -479,60 +480,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(int n, int M, int slic
 }
 
 // ---------------------------------------------------------------------------
-// The choice.  Estimated microseconds of each form on 256 CUs, fitted to
-// sweeps over 17..512 rows x 260..20000 weight rows x k 320..8192 at 4 bits
-// (the other widths differ by a few per cent and keep the order):
-//  tile  4 + groups * 0.125 (UW + 1.5) * rounds, rounds = workgroups / 256
-//        halfway rounded up and at least 1.35 (a lone workgroup per CU has
-//        nothing to overlap its barriers with): 61 us at 512 x 12352 x 2048
-//        (UW 8; 72 at UW 4), 57 us at 512 x 9216 x 2048 (UW 4; 64 at UW 8),
-//        23 us at 300 x 20000 x 512 (UW 4; 32 at UW 8).
-//  split tile  the same over groups / slices, plus the reduction's launch and
-//        its partials' traffic.
-//  deep  4 + stages per wave * rounds * the time of one stage: 17 us at
-//        77 x 2048 x 4096, 12 us at 512 x 513 x 2048, 10 us at 128 x 2048 x
-//        2048.
-struct GemmPlan {
-  enum Form { kTile, kDeep } form;
-  int a, b;  // tile: UW and slices; deep: NT and MT
-};
-
-constexpr int kDeepWaves = 8;
-
-inline int div_up(int a, int b) { return (a + b - 1) / b; }
-
-GemmPlan gemm_plan(int m, int n, int k, size_t part_floats) {
-  const int G = k >> 6;
-  GemmPlan best{GemmPlan::kTile, 4, 1};
-  double least = 1e30;
-  auto take = [&](double t, GemmPlan p) {
-    if (t < least) {
-      least = t;
-      best = p;
-    }
-  };
-  for (int uw : {2, 3, 4, 8})
-    for (int slices = 1; slices <= 16; slices *= 2) {
-      if (slices > 1 && (G / slices < 4 || size_t(slices) * m * n > part_floats)) break;
-      const double r = double(div_up(n, 64)) * div_up(m, 32 * uw) * slices / 256.0;
-      const double whole = double(int64_t(r) + (r > double(int64_t(r)) ? 1 : 0));
-      const double rounds = (r + whole) / 2 > 1.35 ? (r + whole) / 2 : 1.35;
-      double t = 4.0 + div_up(G, slices) * 0.125 * (uw + 1.5) * rounds;
-      if (slices > 1) t += 4.5 + double(m) * n * (slices * 4.0 + 2.0) / 2.5e6;
-      take(t, {GemmPlan::kTile, uw, slices});
-    }
-  struct {
-    int nt, mt;
-    double stage;
-  } const deep[] = {{1, 2, 1.9}, {1, 3, 3.0}, {2, 2, 3.2}, {2, 3, 4.1}, {2, 4, 5.4}};
-  for (const auto& d : deep) {
-    const int blocks = div_up(n, 16 * d.nt) * div_up(m, 16 * d.mt);
-    take(4.0 + double(div_up(div_up(G, 2), kDeepWaves)) * div_up(blocks, 256) * d.stage,
-         {GemmPlan::kDeep, d.nt, d.mt});
-  }
-  return best;
-}
-
 template <int BITS, int UW, bool SPLIT, bool MIX>
 void launch_tile(const QWeight& w, const uint16_t* x, int64_t xs, int m, int per, dim3 grid,
                  const ProjEpilogue& e, hipStream_t s) {
@@ -557,7 +504,8 @@ void launch_gemm(const QWeight& w, const uint16_t* x, int64_t xs, int m, const P
                                       e, s);
     return;
   }
-  const GemmPlan p = gemm_plan(m, w.n, w.k, e.part ? e.part_floats : 0);
+  const GemmPlan p =
+      gemm_plan(m, w.n, w.k, BITS, e.mode == kHcWrite, e.part ? e.part_floats : 0);
   if (p.form == GemmPlan::kDeep) {
     switch (p.a * 10 + p.b) {
       case 12: launch_deep<BITS, 1, 2>(w, x, xs, m, e, s); break;

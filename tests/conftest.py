@@ -1,6 +1,8 @@
 """Shared fixtures: the native library harness and the CPU oracle."""
+import ctypes
 import importlib.util
 import os
+import subprocess
 import sys
 
 import pytest
@@ -36,3 +38,21 @@ def orc():
     from oracle import oracle
 
     return oracle
+
+
+@pytest.fixture(scope="session")
+def gemm_plan(tmp_path_factory):
+    """The form the GEMM beyond 16 rows takes: "T<32-row blocks>.<k slices>" or
+    "D<16-row weight tiles>.<16-row activation tiles>"."""
+    src = os.path.join(ROOT, "tests", "gemm_plan.cpp")
+    so = str(tmp_path_factory.mktemp("plan") / "gemm_plan.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", src, "-o", so], check=True)
+    fn = ctypes.CDLL(so).gemm_plan
+    fn.argtypes = [ctypes.c_int] * 5 + [ctypes.c_size_t, ctypes.c_void_p]
+
+    def plan(m, n, k, bits, streams=False, part_floats=0):
+        out = (ctypes.c_int * 3)()
+        fn(m, n, k, bits, streams, part_floats, out)
+        return f"{'TD'[out[0]]}{out[1]}.{out[2]}"
+
+    return plan

@@ -48,8 +48,15 @@ def blocks(eng, cfg, prompt):
 
 
 @pytest.mark.parametrize("n", [17, 77, 200, 301, 512])
-def test_chunk_layer_matches_blocks(engine, n):
+def test_chunk_layer_matches_blocks(engine, gemm_plan, n):
     eng, cfg = engine
+    # both sides of a layer that split k over workgroups: the low-rank
+    # projection always, the output projection where it is deep and has rows
+    bits, H = cfg["bits"], cfg["hidden"]
+    assert gemm_plan(n, 260, 4 * H, bits, False, 4 << 20) in ("T2.16", "T3.16")
+    deep = cfg["heads"] * cfg["head_dim"] if cfg["attn_every"] == 1 else 128 * cfg["gdn_hv"]
+    out = gemm_plan(n, H, deep, bits, True, 4 << 20)
+    assert (out[0] == "T" and out[-2:] != ".1") == (deep == 4096 and n > 17)
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n)
     want, wids = blocks(eng, cfg, prompt)
     eng.reset(0)
