@@ -733,8 +733,7 @@ __global__ __launch_bounds__(512) void prefill_attn_kernel(
         pl[(4 * kq + r) * kPfVLd + 16 * c + j] = __builtin_bit_cast(uint16_t, __bf16(pv - hf));
       }
     // P is this wave's own; its bf16 stores stay before the 16-byte loads
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     // O += P V: A = P (pair j, keys 32 s + 8 kq ..), B = V^T rows (dim 16 n + j)
 #pragma unroll
     for (int st = 0; st < kPfKeys / 32; ++st) {

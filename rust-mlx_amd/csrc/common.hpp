@@ -34,6 +34,15 @@ MX_HD uint16_t f32_to_bf16(float f) {
 // Round an fp32 value to the nearest bf16 value, keeping fp32 storage.
 MX_HD float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
+// What the lanes of this wave wrote to LDS before, any of its lanes reads after
+// (and the reverse).  A wave barrier alone only holds the instructions in
+// place once they are chosen: without the fence the compiler may still move
+// loads over stores that it takes for other memory.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 MX_HD float fmaf_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // e^x: Cody-Waite reduction x = n*ln2 + r, |r| <= ln2/2, degree-7 Taylor

@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kPrepThreads) void chunk_prep_kernel(
       for (int m = bj; m < bi; ++m)
         acc = mm16(Am + (16 * bi) * kLd + 16 * m, kLd, Tm + (16 * m) * kLd + 16 * bj, kLd, acc);
       store16(tmp[wave], 17, acc, 1.0f);
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       acc = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
       acc = mm16(Tm + (16 * bi) * kLd + 16 * bi, kLd, tmp[wave], 17, acc);
       store16(Tm + (16 * bi) * kLd + 16 * bj, kLd, acc, -1.0f);

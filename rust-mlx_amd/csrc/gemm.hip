@@ -448,7 +448,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(QWeight w, const uint16_
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) out[(4 * kq + r) * kOut + 16 * t + j] = y[t][u][r];
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       const int row = int(blockIdx.x) * 64 + wn * 32 + (lane & 31);
       const int m0 = mb + wm * 16 * UW + 16 * u;
 // two rows at a time: more need more registers than the products do
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(QWeight w, const uint16_
           gemm_epilogue<2>(e, n, M, {m0 + r, m0 + r + 2}, row, {v0, v1});
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
     }
   }
 }
