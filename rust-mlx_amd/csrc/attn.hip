@@ -462,9 +462,10 @@ __global__ __launch_bounds__(kMaxHd) void combine_kernel(const float* __restrict
 
 constexpr int kPfKeys = 64;  // keys per tile of the prefill kernel
 // Keys of one split of a query block that attends to `keys` keys in at most
-// `splits` splits: whole tiles, every split but the last full.
+// `splits` splits: whole tiles, every split but the last full.  One tile for a
+// block without keys (rows at position -1): the combine divides by it.
 __device__ __forceinline__ int prefill_split_len(int keys, int splits) {
-  const int tiles = (keys + kPfKeys - 1) / kPfKeys;
+  const int tiles = max((keys + kPfKeys - 1) / kPfKeys, 1);
   return (tiles + splits - 1) / splits * kPfKeys;
 }
 
@@ -553,7 +554,8 @@ __global__ __launch_bounds__(256) void combine_fast_kernel(const float* __restri
 // The split's (m, l, O) per pair go to o_part / ml_part at chunk index =
 // split, which combine_fast_kernel merges.  Rows of
 // one query block must share a slot (a prefill chunk's rows do).
-// max / sum over the 16 lanes of a row by rotations (no LDS)
+//
+// max / sum over the 16 lanes of a row by rotations (no LDS):
 template <int ROT>
 __device__ __forceinline__ float row_ror(float v) {
   return __builtin_bit_cast(

@@ -149,3 +149,32 @@ def test_attn_prefill_splits_of_every_kind(mx, orc, heads, kv_heads, hd, p0, row
     g = bf(out.numpy()).astype(np.float64)
     scale = np.abs(ref).max(axis=2, keepdims=True)
     assert np.all(np.abs(g - ref) <= 2.0 ** -6 * np.abs(ref) + 2.0 ** -9 * scale)
+
+
+def test_attn_prefill_block_without_keys(mx, orc):
+    """A query block whose rows all lie before the first position attends to
+    nothing (its rows come out as NaN, as in the decode form) and leaves the
+    other blocks' bits alone."""
+    heads, kv_heads, hd, max_ctx, rows = 8, 1, 128, 256, 48
+    rng = np.random.default_rng(3)
+    kc, vc = (orc.f32_to_bf16(rng.standard_normal((1, kv_heads, max_ctx, hd)).astype(np.float32))
+              for _ in range(2))
+    q = orc.f32_to_bf16((rng.standard_normal((rows, heads, hd)) * 0.3).astype(np.float32))
+    qkv = orc.f32_to_bf16(rng.standard_normal((rows, 2 * heads * hd)).astype(np.float32))
+    dims = mx.AttnDimsC(heads, kv_heads, hd, max_ctx, kv_heads * max_ctx * hd)
+    ws = mx.DeviceArray((mx.lib.mx_attn_workspace_bytes(rows, heads, hd, max_ctx),), np.uint8)
+    dq, dqkv, dk, dv = (mx.DeviceArray.from_numpy(a) for a in (q, qkv, kc, vc))
+    dsl = mx.DeviceArray.from_numpy(np.zeros(rows, np.int32))
+    got = []
+    for empty in (False, True):
+        pos = np.arange(100, 100 + rows, dtype=np.int32)
+        if empty:
+            pos[16:32] = -1  # 16 rows to a block at eight q heads per kv head
+        dpos = mx.DeviceArray.from_numpy(pos)
+        out = mx.DeviceArray((rows, heads, hd), np.uint16)
+        mx.check(mx.lib.mx_attn_decode(dq.ptr, dqkv.ptr, 2 * heads * hd, rows, dsl.ptr, dpos.ptr,
+                                       dk.ptr, dv.ptr, C.byref(dims), 3, ws.ptr, out.ptr, None))
+        got.append(out.numpy())
+    live = np.r_[0:16, 32:48]
+    assert (got[0][live] == got[1][live]).all()
+    assert np.isnan(bf(got[1][16:32])).all()
