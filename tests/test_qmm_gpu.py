@@ -127,11 +127,11 @@ def test_moe_experts_mfma_prefill_chunk_rows(mx, orc, rows, E, top_k, H):
 @pytest.mark.parametrize("gbits,dbits,H,I", [(5, 6, 512, 512), (6, 8, 1024, 256),
                                               (8, 4, 512, 768), (4, 5, 256, 1280)])
 def test_moe_experts_mfma_prefill_chunk_widths(mx, orc, gbits, dbits, H, I):
-    """The prefill chunk's expert kernels for every code width (4/8-bit: the
-    32-row tile forms, each lane reading a group's 32 codes of its half with
-    16-byte loads; 5/6-bit: the 16-row forms), at depths of 4..20 groups,
-    against the exact kernels eight rows at a time within the north star's
-    tolerance."""
+    """The prefill chunk's expert kernels for every code width at depths of
+    4..20 groups, against the exact kernels eight rows at a time within the
+    north star's tolerance: depths that are multiples of 512 with the
+    activation rows in LDS, the others in the general forms (every width of
+    those: test_experts_gpu.py)."""
     from test_layers_gpu import Moe
 
     E, top_k, rows = 32, 6, 40
