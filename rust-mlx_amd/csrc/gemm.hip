@@ -314,14 +314,18 @@ __global__ __launch_bounds__(64 * KS) void gemm_deep_kernel(QWeight w,
 // barriers and dequantising with another's matrix-core work.  512 x 12352 x
 // 2048, 4 bits: 61 us (UW = 8), 91 us with two groups per stage at two
 // workgroups per CU.
-// MIX (kHcUpMix): the 64 weight rows are the four streams' rows s H + c of 16
+// KIND: what becomes of the sums.  Each is a kernel of its own: with the other
+// epilogues' code beside it the plain one took 62.6 us at that size.
+// kTileMix (kHcUpMix): the 64 weight rows are the four streams' rows s H + c of 16
 // columns c, mixed through LDS in the epilogue (dense_kernel's arithmetic).
-// SPLIT: fp32 partial sums to e.part, added by gemm_reduce_kernel.
-template <int BITS, int UW, bool SPLIT, bool MIX>
+// kTileSplit: fp32 partial sums to e.part, added by gemm_reduce_kernel.
+enum : int { kTilePlain, kTileSplit, kTileMix, kTileEpilogue };
+template <int BITS, int UW, int KIND>
 __global__ __launch_bounds__(256) void gemm_tile_kernel(QWeight w, const uint16_t* __restrict__ x,
                                                         int64_t x_stride, int M, int per,
                                                         ProjEpilogue e) {
   constexpr int kM = 32 * UW, kLd = 64;
+  constexpr bool MIX = KIND == kTileMix, SPLIT = KIND == kTileSplit;
   __shared__ __align__(16) uint16_t lds[(kM + 2 * 64) * kLd];
   uint16_t* xs = lds;              // [kM][64]
   uint16_t* wh = lds + kM * kLd;   // [64][64]
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(QWeight w, const uint16_
       }
       e.y[size_t(m) * e.y_stride + cb + c] = f32_to_bf16(round_bf16(sum) / 4.0f);
     }
-  } else if (!SPLIT && e.mode == kPlain) {
+  } else if constexpr (KIND == kTilePlain) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int row = int(blockIdx.x) * 64 + wn * 32 + 16 * t + j;
@@ -480,11 +484,11 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(int n, int M, int slic
 }
 
 // ---------------------------------------------------------------------------
-template <int BITS, int UW, bool SPLIT, bool MIX>
+template <int BITS, int UW, int KIND>
 void launch_tile(const QWeight& w, const uint16_t* x, int64_t xs, int m, int per, dim3 grid,
                  const ProjEpilogue& e, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_tile_kernel<BITS, UW, SPLIT, MIX>), grid, dim3(256), 0, s, w, x, xs, m,
-                     per, e);
+  hipLaunchKernelGGL((gemm_tile_kernel<BITS, UW, KIND>), grid, dim3(256), 0, s, w, x, xs, m, per,
+                     e);
 }
 
 template <int BITS, int NT, int MT>
@@ -500,8 +504,8 @@ void launch_gemm(const QWeight& w, const uint16_t* x, int64_t xs, int m, const P
                  hipStream_t s) {
   const int G = w.k >> 6;
   if (e.mode == kHcUpMix) {
-    launch_tile<BITS, 4, false, true>(w, x, xs, m, G, dim3(div_up(e.hidden, 16), div_up(m, 128)),
-                                      e, s);
+    launch_tile<BITS, 4, kTileMix>(w, x, xs, m, G, dim3(div_up(e.hidden, 16), div_up(m, 128)), e,
+                                   s);
     return;
   }
   const GemmPlan p =
@@ -518,16 +522,17 @@ void launch_gemm(const QWeight& w, const uint16_t* x, int64_t xs, int m, const P
   }
   const int per = div_up(G, p.b);
   const dim3 grid(div_up(w.n, 64), div_up(m, 32 * p.a), p.b);
-  switch (p.a * 2 + (p.b > 1 ? 1 : 0)) {
-    case 4: launch_tile<BITS, 2, false, false>(w, x, xs, m, per, grid, e, s); break;
-    case 5: launch_tile<BITS, 2, true, false>(w, x, xs, m, per, grid, e, s); break;
-    case 6: launch_tile<BITS, 3, false, false>(w, x, xs, m, per, grid, e, s); break;
-    case 7: launch_tile<BITS, 3, true, false>(w, x, xs, m, per, grid, e, s); break;
-    case 8: launch_tile<BITS, 4, false, false>(w, x, xs, m, per, grid, e, s); break;
-    case 9: launch_tile<BITS, 4, true, false>(w, x, xs, m, per, grid, e, s); break;
-    case 16: launch_tile<BITS, 8, false, false>(w, x, xs, m, per, grid, e, s); break;
-    default: launch_tile<BITS, 8, true, false>(w, x, xs, m, per, grid, e, s); break;
-  }
+#define MX_TILE(U)                                                            \
+  case U:                                                                     \
+    if (p.b > 1)                                                              \
+      launch_tile<BITS, U, kTileSplit>(w, x, xs, m, per, grid, e, s);         \
+    else if (e.mode == kPlain)                                                \
+      launch_tile<BITS, U, kTilePlain>(w, x, xs, m, per, grid, e, s);         \
+    else                                                                      \
+      launch_tile<BITS, U, kTileEpilogue>(w, x, xs, m, per, grid, e, s);      \
+    break;
+  switch (p.a) { MX_TILE(2) MX_TILE(3) MX_TILE(4) MX_TILE(8) }
+#undef MX_TILE
   if (p.b > 1)
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3(unsigned((size_t(m) * w.n + 255) / 256)),
                        dim3(256), 0, s, w.n, m, p.b, e);

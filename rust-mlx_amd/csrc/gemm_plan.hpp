@@ -22,30 +22,35 @@ inline int div_up(int a, int b) { return (a + b - 1) / b; }
 inline double soft_max(double a, double b) { return std::cbrt(a * a * a + b * b * b); }
 
 // Estimated microseconds on 256 CUs, fitted to sweeps of every form over 17 ..
-// 512 rows x 64 .. 20000 weight rows x k 256 .. 8192 at all widths, with the
-// weights read from memory (a model's layers follow one another: none of its
-// weights are in a cache).  The form this chooses takes 0.7 % longer than the
-// fastest on average over the sweeps, 5 % at the 95th percentile.  Measured
-// against 128-row tiles with k split to 256 workgroups: 2048 x 4096 with the
-// streams' write 19.9 -> 19.8 us at 128 rows and 26.9 -> 25.1 at 256 (tiles, k
-// in eight slices; deep 20.5 and 28.7), 260 x 8192 at 512 23.4 -> 22.3, 513 x
-// 2048 at 512 17.1 -> 12.5, 12352 x 2048 at 512 91.7 -> 63.3.
+// 512 rows x 64 .. 20000 weight rows x k 256 .. 8192 at all widths, once with
+// the weights from memory (a model's layers follow one another: none of its
+// weights are in a cache) and once with one matrix again and again.  The form
+// this chooses takes 0.6 % longer than the fastest on average over the sweeps,
+// 5 % at the 95th percentile.  From memory, against 128-row tiles with k split
+// to 256 workgroups: 2048 x 4096 with the streams' write 26.9 -> 25.0 us at 256
+// rows (tiles, k in eight slices; deep 28.7) and 19.9 both at 128 (deep 20.5),
+// 260 x 8192 at 512 23.4 -> 21.6, 513 x 2048 at 512 17.1 -> 12.5, 12352 x 2048
+// at 512 91.7 -> 61.3.
 //
 // tile: every group costs a workgroup its latency or, with several on a CU,
 // their matrix-core time.
 inline double gemm_tile_us(int m, int n, int k, int bits, bool streams, int uw, int slices) {
-  const int resident = uw == 2 ? 5 : uw == 8 ? 2 : 4;  // workgroups of a CU, by registers
+  // workgroups of a CU, by the registers of the kernel for these outputs
+  const int resident = uw == 2   ? (streams && slices == 1 ? 5 : 6)
+                       : uw == 3 ? (streams || slices > 1 ? 4 : 5)
+                       : uw == 4 ? 4
+                                 : 2;
   const double per_cu = double(div_up(n, 64)) * div_up(m, 32 * uw) * slices / 256.0;
-  const double latency = 0.52 + 0.118 * uw;
-  const double busy = 0.193 + 0.074 * uw + (bits == 4 ? 0.0 : 0.018);
+  const double latency = 0.498 + 0.115 * uw;
+  const double busy = 0.231 + 0.076 * uw + (bits == 4 ? 0.0 : 0.019);
   const double rounds = std::floor(per_cu / resident), rest = per_cu - rounds * resident;
   double group = rounds * soft_max(latency, resident * busy);
   if (rest > 0) group += soft_max(latency, (rest + std::ceil(rest)) / 2 * busy);
   const double outs = double(m) * n * 1e-6;
-  double t = 3.85 + div_up(k >> 6, slices) * group + 0.29 * per_cu * (slices > 1 ? uw : uw / 2.0);
-  if (slices > 1) t += 3.0 + 0.2 * outs * (4 * slices + 2);  // the reduction
+  double t = 3.58 + div_up(k >> 6, slices) * group + 0.261 * per_cu * (slices > 1 ? uw : uw / 2.0);
+  if (slices > 1) t += 5.78 + 0.095 * outs * (4 * slices + 2);  // the reduction
   // kHcWrite reads and writes four streams, here two rows of a wave at a time
-  if (streams) t += 2.5 * outs + (slices > 1 ? 0.0 : 2.5 * uw);
+  if (streams) t += slices > 1 ? 1.61 * outs : 4.14 * outs + 2.82 * uw;
   return t;
 }
 
@@ -56,14 +61,14 @@ inline double gemm_deep_us(int m, int n, int k, int bits, bool streams, int nt, 
   const double groups = double(div_up(n, 16 * nt)) * div_up(m, 16 * mt);
   const double per_cu = groups / 256.0;
   const int rounds = int(std::ceil(per_cu / resident));
-  const double stage = 0.23 + 0.35 * mt + 1.33 * nt + 0.06 * mt * nt;
-  const double two = resident == 2 ? 1.73 : 1.0;  // both workgroups of a CU
+  const double stage = 0.115 + 0.516 * mt + 1.42 * nt + 0.093 * mt * nt;
+  const double two = resident == 2 ? 1.646 : 1.0;  // both workgroups of a CU
   const double walk = div_up(div_up(G, 2), kDeepWaves) * stage *
                       ((rounds - 1) * two + (per_cu - (rounds - 1) * resident > 1 ? two : 1.0));
-  const double read = double(n) * k * (bits / 8.0 + 0.0625) / 14.1e6 +
-                      groups * G * (2048.0 * mt + 128.0 * nt * bits) / 8.0e6;
-  const double t = 1.36 + std::sqrt(std::sqrt(walk * walk * walk * walk + read * read * read * read));
-  return streams ? t + 1.3 + 3.4e-6 * m * n : t;
+  const double read = double(n) * k * (bits / 8.0 + 0.0625) / 13.1e6 +
+                      groups * G * (2048.0 * mt + 128.0 * nt * bits) / 10.2e6;
+  const double t = 0.71 + std::sqrt(std::sqrt(walk * walk * walk * walk + read * read * read * read));
+  return streams ? t + 2.47 + 2.33e-6 * m * n : t;
 }
 
 // m activation rows, weights n x k; streams: the kHcWrite epilogue;
