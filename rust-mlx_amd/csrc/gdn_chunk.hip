@@ -91,8 +91,8 @@ __device__ __forceinline__ void store16(float* Z, int ldz, floatx4_t v, float sc
 // operands swapped): transposed it is four consecutive k per lane, as it is
 // stored; untransposed its registers are the A operand of P W.  72 KB of LDS
 // (V takes A's place once T is known): two workgroups per CU.  Bound by the
-// serial inverse and the barriers between its steps; at 32 heads x 32 chunks
-// 52 us, 159 us with four waves, the scales formed per product and every
+// serial inverse and the barriers between its steps (matrix cores 35 % busy); at
+// 32 heads x 32 chunks 50 us, 159 us with four waves, the scales formed per product and every
 // result stored one float per lane.
 __global__ __launch_bounds__(kPrepThreads) void chunk_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
@@ -302,11 +302,13 @@ __global__ __launch_bounds__(kPrepThreads) void chunk_prep_kernel(
 // read the state that enters the chunk.  State and D lie in LDS by column, so
 // an operand is sixteen bytes per lane; both copies of the state alternate, so
 // a chunk takes two barriers.  Operands are requested a chunk ahead (they do
-// not depend on the state).  At 32 heads x 32 chunks 114 us, 3.6 us a chunk,
-// 213 us with one wave per SIMD doing both, the output after D.  Bound by the
-// workspace's way from L2 (every slice reads 98 KB a chunk: 89 us with chunk
-// 0's operands throughout; fp32 K'^T and all of P cost 14 us, slices of a head
-// on different XCDs 16 us) and by the chain's two barriers and 64 fp32 MFMAs.
+// not depend on the state).  At 32 heads x 32 chunks 104 us, 3.25 us a chunk,
+// 213 us with one wave per SIMD doing both, the output after D.  Bound by fp32
+// matrix-core time (46 % of the cycles: 64 products of 32 cycles on each SIMD for
+// the chain and 48 for the outputs of a chunk), by the chain's two barriers and by
+// the workspace's way from L2 (every slice reads 98 KB a chunk; with chunk 0's
+// operands throughout a form of 114 us took 89; fp32 K'^T and all of P cost 14 us,
+// slices of a head on different XCDs 16 us).
 __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(
     const float* __restrict__ ws, int hv, int t, int nchunks, const int32_t* __restrict__ slots,
     float* __restrict__ state, uint16_t* __restrict__ y) {

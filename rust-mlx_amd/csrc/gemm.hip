@@ -223,8 +223,9 @@ __device__ __forceinline__ void gemm_epilogue(const ProjEpilogue& e, int n, int 
 // leaves the last stage's quarters 2 and 3 empty: both operands are zero.
 // Bound by the latency of a wave's few stages; splitting k over the waves
 // instead of walking it in one keeps 2048 waves busy on 128 output tiles.
-// 77 x 2048 x 4096, 4 bits: 16.9 us, 66.8 us with one workgroup per 64
-// weight rows walking all of k.
+// 77 x 2048 x 4096, 4 bits: 15.9 us, 66.8 us with one workgroup per 64
+// weight rows walking all of k (weights in a cache; the k split over workgroups,
+// where there is room for its sums, 17.7 with the streams' write, 19.5 here).
 template <int BITS, int NT, int MT, int KS>
 __global__ __launch_bounds__(64 * KS) void gemm_deep_kernel(QWeight w,
                                                             const uint16_t* __restrict__ x,

@@ -469,11 +469,17 @@ __global__ __launch_bounds__(64 * T * KS) void xq_dense_kernel(QWeight w,
 // every 64 weight rows and meets three times for each.  Bound by the weight
 // stream: 8 rows x 151936 x 2048, 8 bits 66.3 us (5.0 TB/s), 109.8 before; 4
 // bits 47.0 (87.4), 6 bits 62.6 (107.4).
-constexpr int kLongWaves = 8, kLongPerCu = 2;  // 69 KB of LDS, 94-122 registers
+constexpr int kLongWaves = 8, kLongPerCu = 2;  // 71 KB of LDS, 94-122 registers
 // More rows than one round of xq_dense_kernel's 64-row workgroups (one fits a
 // CU) covers.  16000 rows of 4 bits: 8.4 / 10.3 us there (1 / 8 activation
 // rows), 11.2 / 15.0 here; 20000: 13.4 / 17.7 there, 11.4 / 15.4 here (6 bits
-// 15.8 / 21.2 and 14.5 / 18.5, 8 bits 15.3 / 20.3 and 11.6 / 15.6).
+// 15.8 / 21.2 and 14.5 / 18.5, 8 bits 15.3 / 20.3 and 11.6 / 15.6).  Only at k =
+// 2048: shallower rows are digitised in less time than their weights take, and
+// 20000 rows of k = 1024 take 8.2 / 10.2 us there and 8.0 / 9.7 here (6 bits 9.8
+// / 11.8 and 9.9 / 11.6, 8 bits 9.1 / 11.7 and 8.3 / 10.0), k = 512 5.4 / 6.9 and
+// 5.7 / 6.6, k = 256 4.0 / 4.9 and 4.2 / 4.7: a tenth either way for nine more
+// kernels (151936 rows of k = 1024: 25.3 / 34.2 and 22.3 / 27.1).  Deeper rows'
+// operands leave room in LDS for one workgroup per CU.
 constexpr int kLongRows = 256 * 64;
 
 template <int BITS, int SPW, bool RM>
